@@ -88,7 +88,11 @@ typedef struct sodecl_options {
     int verbose;             /* print "Compute results runtime" like the reference */
     size_t traj_budget_bytes;/* device trajectory buffer budget; 0 = 8 GiB */
     int pairwise;            /* group schedule with a plugin that defines the pairwise drift (sode_pair,
-                                sode_system_pairsum): 0 = automatic (the full N x (N+1) LDS matrix when
+                                sode_system_pairsum): 0 = automatic (in the default arithmetic the plugin's
+                                field form, sode_field and sode_system_field, when it has one: the coupling
+                                through sums of per-component features, at most 16 components per lane, an
+                                orbit on the whole group or, with group_size 0, on the part of it that is
+                                estimated fastest; else the full N x (N+1) LDS matrix when
                                 the group has two lanes per component and the matrix is at most 16 KiB
                                 per orbit, else lane exchange when the group has a lane per component,
                                 else the full matrix while it fits, else off), 1 = always (lane exchange, else half

@@ -21,7 +21,7 @@
 //     gx[i] = sum_k lam[k] df_k/dx_i for this lane's components
 //             i = sodecl_lane() + c * sodecl_group_size();
 //     gp[k] += sum_i lam[i] df_i/dp_k, every entry updated by one lane only.
-#if SODECL_SCHEDULE == 2 && defined(SODECL_ADJOINT) && SODECL_HAS_VJP_GROUP && \
+#if SODECL_SCHEDULE == 2 && !SODECL_USE_FIELD && defined(SODECL_ADJOINT) && SODECL_HAS_VJP_GROUP && \
     (SODECL_SOLVER == 1 || SODECL_SOLVER == 2)
 
 // One VJP through LDS: publish point v and cotangent l, barrier, evaluate.

@@ -22,6 +22,7 @@
 //                 l, l+G, ...; stage vectors are staged in LDS and every lane
 //                 evaluates its components through the plugin's per-component
 //                 entry point (coupled systems such as Kuramoto)
+//                 (systems with a field form: field.hip instead)
 //   sodecl_team   SODECL_GROUP lanes per orbit, each with the whole state;
 //                 the plugin's team entry point shares the costly terms
 // All run many ksteps segments per launch and write the snapshot that
@@ -92,11 +93,10 @@ SODECL_INLINE sodecl_u64 sodecl_counter_word(double c)
 // One Box-Muller pair scaled by sqrt(dt) (stochastic_solver_caller.cl:54-65),
 // with the logarithm, sine and cosine specialised to the uniforms' ranges
 // (gauss.hip).
-SODECL_INLINE void sodecl_noise_pair(int orbit, double counter, double dtsqrt, double* z0, double* z1)
+SODECL_INLINE void sodecl_noise_pair(int orbit, sodecl_u64 word, double dtsqrt, double* z0, double* z1)
 {
     sodecl_u64 w0, w1;
-    sodecl_threefry2x64_20((sodecl_u64)orbit, sodecl_counter_word(counter), SODECL_RNG_KEY0, SODECL_RNG_KEY1,
-                           &w0, &w1);
+    sodecl_threefry2x64_20((sodecl_u64)orbit, word, SODECL_RNG_KEY0, SODECL_RNG_KEY1, &w0, &w1);
     const double u0 = sodecl_u01(w0);
     const double u1 = sodecl_u01(w1);
     const double r = sqrt(-2 * sodecl_log_positive(u0));
@@ -323,7 +323,7 @@ SODECL_INLINE void sodecl_lane_orbit(int i, double* __restrict__ t_state, double
                 int nc = 0;
                 for (int in = 0; in < calls; ++in) {
                     double z0, z1;
-                    sodecl_noise_pair(i, cnt, dtsqrt, &z0, &z1);
+                    sodecl_noise_pair(i, sodecl_counter_word(cnt), dtsqrt, &z0, &z1);
                     cnt = cnt + 1;
                     if (nc < _numnoi_) noise[nc++] = z0;
                     if (nc < _numnoi_) noise[nc++] = z1;
@@ -471,7 +471,7 @@ sodecl_team(double* __restrict__ t_state, double* __restrict__ y_state, const do
 // Rows are double-buffered so one barrier per stage suffices.  (The group
 // never spans wavefronts, so no barrier waits on another wavefront.)
 // ---------------------------------------------------------------------------
-#if SODECL_SCHEDULE == 2 && SODECL_HAS_COMPONENT && !SODECL_IS_IMPLICIT && (!SODECL_IS_SDE || SODECL_HAS_STOCH_COMPONENT)
+#if SODECL_SCHEDULE == 2 && !SODECL_USE_FIELD && SODECL_HAS_COMPONENT && !SODECL_IS_IMPLICIT && (!SODECL_IS_SDE || SODECL_HAS_STOCH_COMPONENT)
 
 #define SODECL_G SODECL_GROUP
 #define SODECL_CPL ((_numeq_ + SODECL_G - 1) / SODECL_G)
@@ -845,7 +845,7 @@ sodecl_group(double* __restrict__ t_state, double* __restrict__ y_state, const d
                         const int nb = k < calls ? buf : (buf ^ 1);
                         const int kk = k < calls ? k : k - calls;
                         double z0, z1;
-                        sodecl_noise_pair(orbit, cnt + (double)k, dtsqrt, &z0, &z1);
+                        sodecl_noise_pair(orbit, sodecl_counter_word(cnt + (double)k), dtsqrt, &z0, &z1);
                         if (2 * kk < _numnoi_) sh_n[nb][slot][2 * kk] = z0;
                         if (2 * kk + 1 < _numnoi_) sh_n[nb][slot][2 * kk + 1] = z1;
                     }

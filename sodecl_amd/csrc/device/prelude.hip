@@ -1,13 +1,15 @@
 // Device helpers visible to the system plugin (emitted before it).
 
 // A double moved across lanes by one DPP control (two 32-bit moves); a lane
-// whose source lies outside the wavefront receives 0.
+// whose source lies outside its row or the wavefront, or is not active,
+// receives 0 (the instruction's own bound control: no register has to hold
+// the 0 beforehand, which cost a move per 32-bit half).
 template <int CTRL>
 __device__ inline double sodecl_dpp(double v)
 {
     const long long bits = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_update_dpp(0, (int)(bits & 0xffffffffll), CTRL, 0xF, 0xF, false);
-    const int hi = __builtin_amdgcn_update_dpp(0, (int)(bits >> 32), CTRL, 0xF, 0xF, false);
+    const int lo = __builtin_amdgcn_mov_dpp((int)(bits & 0xffffffffll), CTRL, 0xF, 0xF, true);
+    const int hi = __builtin_amdgcn_mov_dpp((int)(bits >> 32), CTRL, 0xF, 0xF, true);
     return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned int)lo);
 }
 #define SODECL_DPP_XOR1 0xB1          // quad_perm [1,0,3,2]
@@ -43,34 +45,46 @@ __device__ inline void sodecl_wave_sync()
 #if SODECL_SCHEDULE == 2
 __device__ inline int sodecl_group_size() { return SODECL_GROUP; }
 __device__ inline int sodecl_lane() { return (int)(threadIdx.x % SODECL_GROUP); }
-// Reduction over the group in levels of lane distance 1, 2, 4, 8, 16, 32.
-// The first four are DPP moves inside a 16-lane row: xor 1 and xor 2 by quad
-// permutations, then the half-row and row mirrors, which pair every lane with
-// the opposite block of the previous level (whose lanes all hold the same
-// partial sum) exactly as xor 4 and xor 8 would; the last two are cross-lane
-// permutes.  At every level the two partners add the same two numbers, so
-// every lane ends with a bit-identical sum.
-// A group of the whole wavefront reads the four row sums into scalar
-// registers instead (v_readlane) and adds them as (r0 + r1) + (r2 + r3):
-// the same two levels of additions on the same operands, without the
-// permutes.
-__device__ inline double sodecl_readlane(double v, int lane)
+// Reduction over aligned blocks of W lanes in levels of lane distance 1, 2,
+// 4, 8, 16, 32.  The first four are DPP moves inside a 16-lane row: xor 1 and
+// xor 2 by quad permutations, then the half-row and row mirrors, which pair
+// every lane with the opposite block of the previous level (whose lanes all
+// hold the same partial sum) exactly as xor 4 and xor 8 would.  The last two
+// swap rows (v_permlane16_swap) or half wavefronts (v_permlane32_swap) of two
+// copies of the value, one register per 32-bit half: the copies then hold one
+// partner's sum each on both partners.  At every level the two partners add
+// the same two numbers, so every lane ends with a bit-identical sum.
+__device__ inline double sodecl_swapped_sum(double v, bool rows)
 {
     const long long bits = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_readlane((int)(bits & 0xffffffffll), lane);
-    const int hi = __builtin_amdgcn_readlane((int)(bits >> 32), lane);
-    return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned int)lo);
+    const int l = (int)(bits & 0xffffffffll), h = (int)(bits >> 32);
+    const auto lo = rows ? __builtin_amdgcn_permlane16_swap(l, l, false, false)
+                         : __builtin_amdgcn_permlane32_swap(l, l, false, false);
+    const auto hi = rows ? __builtin_amdgcn_permlane16_swap(h, h, false, false)
+                         : __builtin_amdgcn_permlane32_swap(h, h, false, false);
+    return __longlong_as_double(((long long)(int)hi[0] << 32) | (long long)(unsigned int)lo[0]) +
+           __longlong_as_double(((long long)(int)hi[1] << 32) | (long long)(unsigned int)lo[1]);
+}
+// Several sums at once, level by level.
+template <int W, int K>
+__device__ inline void sodecl_lane_sums(double (&v)[K])
+{
+#define SODECL_LANE_LEVEL(LANES, SUM)                             \
+    if (W >= LANES)                                               \
+        _Pragma("unroll") for (int k = 0; k < K; ++k) v[k] = SUM;
+    SODECL_LANE_LEVEL(2, v[k] + sodecl_dpp<SODECL_DPP_XOR1>(v[k]))
+    SODECL_LANE_LEVEL(4, v[k] + sodecl_dpp<SODECL_DPP_XOR2>(v[k]))
+    SODECL_LANE_LEVEL(8, v[k] + sodecl_dpp<SODECL_DPP_HALF_MIRROR>(v[k]))
+    SODECL_LANE_LEVEL(16, v[k] + sodecl_dpp<SODECL_DPP_MIRROR>(v[k]))
+    SODECL_LANE_LEVEL(32, sodecl_swapped_sum(v[k], true))
+    SODECL_LANE_LEVEL(64, sodecl_swapped_sum(v[k], false))
+#undef SODECL_LANE_LEVEL
 }
 __device__ inline double sodecl_group_sum(double v)
 {
-    if (SODECL_GROUP >= 2) v += sodecl_dpp<SODECL_DPP_XOR1>(v);
-    if (SODECL_GROUP >= 4) v += sodecl_dpp<SODECL_DPP_XOR2>(v);
-    if (SODECL_GROUP >= 8) v += sodecl_dpp<SODECL_DPP_HALF_MIRROR>(v);
-    if (SODECL_GROUP >= 16) v += sodecl_dpp<SODECL_DPP_MIRROR>(v);
-    if (SODECL_GROUP == 64)
-        return (sodecl_readlane(v, 0) + sodecl_readlane(v, 16)) + (sodecl_readlane(v, 32) + sodecl_readlane(v, 48));
-    if (SODECL_GROUP >= 32) v += __shfl_xor(v, 16, SODECL_GROUP);
-    return v;
+    double s[1] = {v};
+    sodecl_lane_sums<SODECL_GROUP>(s);
+    return s[0];
 }
 #define SODECL_GROUP_API 1
 #endif

@@ -77,6 +77,9 @@ PluginFeatures detect_features(const std::string& source)
     f.jacobian_band_i = defines("calc_jacobian_band_i");
     f.vjp_group = defines("sode_system_vjp_group");
     f.pairs = defines("sode_pair") && defines("sode_system_pairsum");
+    f.field = defines("sode_field") && defines("sode_system_field") && defines("sode_field_own_param");
+    f.stoch_own = defines("sode_system_stoch_own");
+    f.field_vjp = defines("sode_field_vjp_sum") && defines("sode_field_vjp") && defines("sode_field_vjp_params");
     f.team = defines("sode_system_team");
     f.jacobian_params = defines("calc_jacobian_params");
     f.jacobian_exact = defines("calc_jacobian_exact");
@@ -116,9 +119,9 @@ std::string epsilon_define(const ProgramKey& k)
     return buf;
 }
 
-// sin() and exp() of the system source resolve to sodecl_sin (device/sin.hip)
-// and sodecl_exp (device/exp.hip) unless the caller asked for the device
-// library's; the solver templates after the system source keep the library's
+// sin(), sincos() and exp() of the system source resolve to sodecl_sin
+// (device/sin.hip), sodecl_sincos (device/sincos.hip) and sodecl_exp
+// (device/exp.hip) unless the caller asked for the device library's; the solver templates after the system source keep the library's
 // functions.
 // Text around the user's system source: the own sine and exponential in
 // place of the library's, and in the default arithmetic (fp_contract = 0)
@@ -128,14 +131,14 @@ std::string epsilon_define(const ProgramKey& k)
 // correctly rounded one, the same size of rounding change as contraction).
 std::string system_begin(const ProgramKey& k)
 {
-    return std::string(k.library_sin ? "" : "#define sin sodecl_sin\n") +
+    return std::string(k.library_sin ? "" : "#define sin sodecl_sin\n#define sincos sodecl_sincos\n") +
            (k.library_exp ? "" : "#define exp sodecl_exp\n") +
            (k.fp_contract ? "" : "#pragma clang fp reciprocal(on)\n");
 }
 std::string system_end(const ProgramKey& k)
 {
     return std::string(k.fp_contract ? "" : "#pragma clang fp reciprocal(off)\n") +
-           (k.library_sin ? "" : "#undef sin\n") + (k.library_exp ? "" : "#undef exp\n");
+           (k.library_sin ? "" : "#undef sin\n#undef sincos\n") + (k.library_exp ? "" : "#undef exp\n");
 }
 
 std::string assemble_program(const std::string& system_source, const ProgramKey& k, const PluginFeatures& f)
@@ -168,6 +171,9 @@ std::string assemble_program(const std::string& system_source, const ProgramKey&
     o << "#define SODECL_HAS_JACOBIAN_PARAMS " << (f.jacobian_params ? 1 : 0) << "\n";
     o << "#define SODECL_HAS_JACOBIAN_EXACT " << (f.jacobian_exact ? 1 : 0) << "\n";
     o << "#define SODECL_USE_PAIRS " << (k.schedule == 2 && f.pairs ? k.use_pairs : 0) << "\n";
+    if (k.field_lanes > 0)
+        o << "#define SODECL_USE_FIELD 1\n#define SODECL_FIELD_API 1\n#define SODECL_FL " << k.field_lanes
+          << "\n#define SODECL_FC " << k.field_cpl << "\n#define SODECL_FBLOCK " << k.field_block << "\n";
     if (k.one_wave_per_simd) o << "#define SODECL_KERNEL_ATTR __attribute__((amdgpu_waves_per_eu(1, 1)))\n";
     o << k.extra_defines;
     // OpenCL C spellings a system source may use
@@ -185,6 +191,14 @@ std::string assemble_program(const std::string& system_source, const ProgramKey&
     o << "#line 1 \"system.cl\"\n";
     o << system_source << "\n";
     o << system_end(k);
+    if (k.field_lanes > 0 && !k.library_sin) {
+        // the same source once more, its sincos() marking what it does not
+        // cover instead of branching to the library (device/field.hip)
+        o << "#define SODECL_FIELD_MARKED 1\nnamespace sodecl_marked {\n";
+        o << "#define sin sodecl_sin\n#define sincos sodecl_sincos_marked\n"
+          << (k.library_exp ? "" : "#define exp sodecl_exp\n") << "#pragma clang fp reciprocal(on)\n";
+        o << "#line 1 \"system.cl\"\n" << system_source << "\n" << system_end(k) << "}\n";
+    }
     o << "#pragma clang force_cuda_host_device end\n";
     o << "#line 1 \"integrators.hip\"\n";
     o << kIntegratorsSource << "\n";

@@ -121,7 +121,13 @@ ProgramKey make_key(const sodecl_ctx* ctx, int schedule, int group, int block, c
     // parallelism, and the dispatcher cannot stack two of the waves on one
     // SIMD while another idles (measured: 2x on 65536-orbit RK4 at block
     // sizes of 128 and 512 lanes).
-    const long lanes = (long)ctx->orbits * (schedule == 2 || schedule == 4 ? std::max(group, 1) : 1);
+    FieldConfig field;
+    const bool in_field = field_config(ctx, schedule, group, &field);
+    const int per_orbit = in_field ? field.lanes : schedule == 2 || schedule == 4 ? std::max(group, 1) : 1;
+    const long lanes = (long)ctx->orbits * per_orbit;
+    k.field_lanes = field.lanes;
+    k.field_cpl = field.cpl;
+    k.field_block = field.block;
     k.one_wave_per_simd = (lanes + 63) / 64 <= 4L * device_cus(ctx) ? 1 : 0;
     k.extra_defines = extra;
     return k;
@@ -348,6 +354,64 @@ LaunchCfg choose_config(const sodecl_ctx* c)
     return cfg;
 }
 
+}  // namespace
+
+namespace sodecl_amd {
+
+// The field form replaces the automatic pairwise choice (pairwise = 0) of the
+// default arithmetic: it sums the coupling through the components' features,
+// the strict arithmetic and the explicit pairwise layouts keep the pair terms.
+// A plugin with a group VJP takes it only if it has the field form's VJP too
+// (the adjoint recomputes the forward's own steps).
+//
+// Lanes per orbit: an explicit or tuned group size is taken as it is.
+// Otherwise the power of two with the least estimated time of one drift, the
+// wavefronts of the fullest SIMD times what one wavefront takes: a fixed part
+// (the sums over lanes) and a part per component.  Measured on gfx950 for
+// the sine coupling (16384 orbits of 64 components, nanoseconds per wavefront
+// and drift): 186, 286 and 491 with 1, 2 and 4 components per lane, so 85
+// plus 100 per component; the stochastic form's noise adds about 230 per
+// component.  More than five components per lane run out of registers (eight:
+// 992, with spills) and are taken only where 64 lanes leave no choice.  The
+// fullest SIMD counts: 1500 orbits of 33 components are 1.5 wavefronts per SIMD
+// on 64 lanes and 0.73 on 32, 0.50 against 0.41 ms over 300 RK4 steps.
+bool field_config(const sodecl_ctx* c, int schedule, int group, FieldConfig* f)
+{
+    *f = FieldConfig{};
+    if (schedule != SODECL_SCHEDULE_GROUP || !c->features.field || c->opts.pairwise != 0 || c->opts.fp_contract)
+        return false;
+    const bool sde = c->solver == SODECL_STOCHASTIC_EULER;
+    if (!sde && c->solver != SODECL_EULER && c->solver != SODECL_RUNGE_KUTTA) return false;
+    if (sde && !(c->features.stoch_own && c->nnoi == c->neq)) return false;
+    if (c->features.vjp_group && !c->features.field_vjp) return false;
+    auto cpl = [&](int lanes) {
+        const int n = (c->neq + lanes - 1) / lanes;
+        return sde && (n > 1 || lanes == 1) ? (n + 1) / 2 * 2 : n;   // a noise pair belongs to one lane or two
+    };
+    int lanes = group;
+    if (c->opts.group_size <= 0 && !c->tuned_schedule && !c->tuning) {
+        const long simds = 4L * device_cus(c), per_component = sde ? 330 : 100;
+        auto cost = [&](int l) {
+            const long waves = ((long)c->orbits * l + 63) / 64;
+            return (waves + simds - 1) / simds * (85 + per_component * cpl(l));
+        };
+        lanes = std::min(group, default_group(c->neq));
+        for (int l = lanes / 2; l >= 1 && cpl(l) <= 5; l /= 2)
+            if (cost(l) < cost(lanes)) lanes = l;
+    }
+    if (cpl(lanes) > 16) return false;
+    int block = 256;
+    while (block > std::max(lanes, 64) && ((long)c->orbits * lanes + block - 1) / block < device_cus(c)) block /= 2;
+    f->lanes = lanes;
+    f->cpl = cpl(lanes);
+    f->block = block;
+    return true;
+}
+
+}  // namespace sodecl_amd
+
+namespace {
+
 // Enqueues one launch of the chosen schedule: segments [s0, s0 + nseg) of the
 // trajectory buffer traj (snapshot rows), final snapshot when final_snap.
 int enqueue(sodecl_ctx* c, const LaunchCfg& cfg, double* t, double* y, const double* p, double* cnt, double* traj,
@@ -357,13 +421,20 @@ int enqueue(sodecl_ctx* c, const LaunchCfg& cfg, double* t, double* y, const dou
 {
     auto prog = get_program(c, cfg.schedule, cfg.group, cfg.block);
     if (!prog) return 0;
-    const char* kname = cfg.schedule == 2 ? "sodecl_group" : (cfg.schedule == 4 ? "sodecl_team" : "sodecl_lane");
+    FieldConfig field;
+    const bool in_field = field_config(c, cfg.schedule, cfg.group, &field);
+    const char* kname = in_field ? "sodecl_field"
+                                 : cfg.schedule == 2 ? "sodecl_group" : (cfg.schedule == 4 ? "sodecl_team" : "sodecl_lane");
     hipFunction_t fn = prog->get(kname);
     if (!fn) return fail(c, std::string("kernel ") + kname + " missing from the program");
     // the first norbits orbits only (the rest are the host share's)
     int orbits = norbits >= 0 ? norbits : c->orbits;
-    unsigned grid;
-    if (cfg.schedule == 2 || cfg.schedule == 4) {
+    unsigned grid, block = (unsigned)cfg.block;
+    if (in_field) {
+        const int opb = field.block / field.lanes;
+        grid = (unsigned)((orbits + opb - 1) / opb);
+        block = (unsigned)field.block;
+    } else if (cfg.schedule == 2 || cfg.schedule == 4) {
         const int opb = cfg.block / cfg.group;
         grid = (unsigned)((orbits + opb - 1) / opb);
     } else {
@@ -376,7 +447,7 @@ int enqueue(sodecl_ctx* c, const LaunchCfg& cfg, double* t, double* y, const dou
     }
     void* args[] = {&t, &y, (void*)&p, &cnt, &traj, &newton, &orbits, &s0, &nseg, &final_snap,
                     &ckpt_t, &ckpt_y, &ckpt_every, &gstep0, &stage_ws, &ws_steps};
-    if (!hip_ok(c, hipModuleLaunchKernel(fn, grid, 1, 1, (unsigned)cfg.block, 1, 1, 0, stream, args, nullptr),
+    if (!hip_ok(c, hipModuleLaunchKernel(fn, grid, 1, 1, block, 1, 1, 0, stream, args, nullptr),
                 "hipModuleLaunchKernel"))
         return 0;
     c->used_schedule = cfg.schedule;
@@ -805,6 +876,11 @@ int autotune(sodecl_ctx* c)
         return 0;
     }
     std::ostringstream rep;
+    struct Tuning {   // group sizes are the candidates' own while it lasts
+        sodecl_ctx* c;
+        explicit Tuning(sodecl_ctx* ctx) : c(ctx) { c->tuning = true; }
+        ~Tuning() { c->tuning = false; }
+    } timing(c);
     float best = 1e30f;
     LaunchCfg best_cfg{0, 0, 0};
     for (const LaunchCfg& cfg : tune_candidates(c)) {

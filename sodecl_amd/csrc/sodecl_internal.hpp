@@ -24,6 +24,9 @@ struct PluginFeatures {
     bool jacobian_band_i = false;   // calc_jacobian_band_i(i, y, p, *lower, *diag, *upper)
     bool vjp_group = false;         // sode_system_vjp_group(...) (adjoint, group schedule)
     bool pairs = false;             // sode_pair + sode_system_pairsum (antisymmetric pairwise drift)
+    bool field = false;             // sode_field + sode_system_field (coupling through sums over all components)
+    bool stoch_own = false;         // sode_system_stoch_own (own state and own noise only)
+    bool field_vjp = false;         // sode_field_vjp* + sode_field_own_param (adjoint in field form)
     bool team = false;              // sode_system_team(...) (team schedule)
     bool jacobian_params = false;   // calc_jacobian_params(y, jp[neq][npar], p) (implicit adjoint)
     bool jacobian_exact = false;    // calc_jacobian_exact(y, jac[neq][neq], p) (implicit adjoint)
@@ -44,6 +47,9 @@ struct ProgramKey {
     int newton_max_iter = 1000;
     double newton_tol = 0.0;     // > 0: _epsilon1_ in place of the reference's 1e-07
     int fp_contract = 0;
+    int field_lanes = 0;         // group schedule in field form: lanes per orbit (0: not in field form),
+    int field_cpl = 0;           //   components per lane
+    int field_block = 0;         //   and threads per block of its kernels
     int use_pairs = 0;           // pairwise drift under the group schedule: 0 off, 1 full matrix, 2 half storage
     int one_wave_per_simd = 0;   // the launch has at most one wavefront per SIMD (occupancy hint)
     int library_sin = 0;         // sin() in the system source: 0 sodecl_sin, 1 the device library's
@@ -151,6 +157,7 @@ struct sodecl_ctx {
     // programs: one per (schedule, group, block)
     std::map<std::string, std::shared_ptr<sodecl_amd::Program>> programs;
     int used_schedule = 0, used_group = 0, used_block = 0;
+    bool tuning = false;            // the autotuner is timing its candidates
     // autotuner result (schedule, group, block); tuned_schedule 0 = none
     int tuned_schedule = 0, tuned_group = 0, tuned_block = 0;
     std::string tune_report;
@@ -185,6 +192,13 @@ namespace sodecl_amd {
 int fail(sodecl_ctx* ctx, const std::string& msg);
 ProgramKey make_key(const sodecl_ctx* ctx, int schedule, int group, int block, const std::string& extra);
 bool hip_ok(sodecl_ctx* ctx, hipError_t e, const char* what);
+// The group schedule's field form (device/field.hip) for a group size: lanes
+// per orbit, components per lane and threads per block of its kernels.  False
+// when the context's runs do not take it.
+struct FieldConfig {
+    int lanes = 0, cpl = 0, block = 0;
+};
+bool field_config(const sodecl_ctx* c, int schedule, int group, FieldConfig* f);
 // Program for the given schedule on the context's device (compiled on first use).
 std::shared_ptr<Program> get_program(sodecl_ctx* ctx, int schedule, int group, int block,
                                      const std::string& extra_defines = std::string());

@@ -19,6 +19,10 @@
  *   sode_system_pairsum  the same drift in pairwise form: the pair term
  *                        sin(y_j - y_i) is exactly antisymmetric, so the
  *                        integrator evaluates each pair once;
+ *   sode_field,
+ *   sode_system_field    the same drift through the mean fields of sin y and
+ *                        cos y (O(N) per drift); sode_system_stoch_own and
+ *                        the sode_field_vjp functions go with it;
  *   sode_system_stoch_i  one component of the diffusion term;
  *   calc_jacobian        dense df/dy (implicit solvers, sensitivity checks);
  *   calc_jacobian_params dense df/dp (sensitivity checks).
@@ -151,5 +155,64 @@ void sode_system_vjp_group(double t, double x[_numeq_], double lam[_numeq_], dou
     {
         gp[0] = gp[0] + (A * D - B * C) / (double)(KURA_N);
     }
+}
+#endif
+
+#ifdef SODECL_FIELD_API
+/* Field form: sin(y_j - y_i) = sin y_j cos y_i - cos y_j sin y_i, so with
+ * S = sum_j sin y_j and C = sum_j cos y_j
+ *   f_i = (K/N) (S cos y_i - C sin y_i) + w_i.
+ * The rounding of S and C is about N eps, that of f_i's coupling about K eps:
+ * the same size as the rounding of w_i and below that of the states (which
+ * grow with t), so trajectories keep the accuracy of the pairwise sums. */
+#define SODE_FIELDS 2
+/* K is shared, w_i and (SDE form) the noise amplitude are component i's own. */
+#define SODE_FIELD_SHARED 1
+#define SODE_FIELD_OWN (_numnoi_ > 0 ? 2 : 1)
+int sode_field_own_param(int i, int k)
+{
+    return k == 0 ? i + 1 : _numpar_ - _numnoi_ + i;
+}
+
+void sode_field(int i, double t, double yi, double ps[], double po[], double phi[])
+{
+    sincos(yi, &phi[0], &phi[1]);
+}
+
+double sode_system_field(int i, double t, double yi, double ps[], double po[], double phi[], double sum[])
+{
+    const double s = sum[0] * phi[1] - sum[1] * phi[0];
+    return s * (double)(ps[0] / (double)(KURA_N)) + po[0];
+}
+
+double sode_system_stoch_own(int i, double t, double yi, double ps[], double po[], double zi)
+{
+    return po[1] * zi;
+}
+
+/* The products of the adjoint: sbar_k = sum_i lam_i df_i/dS_k with
+ * df_i/dS = (K/N) cos y_i and df_i/dC = -(K/N) sin y_i; component i's
+ * lam_i df_i/dy_i + sum_k sbar_k dphi_k/dy_i; lam_i df_i/dK for the shared
+ * parameter K and lam_i df_i/dw_i = lam_i for the component's own w_i. */
+void sode_field_vjp_sum(int i, double t, double yi, double ps[], double po[], double phi[], double sum[], double lam,
+                        double sbar[])
+{
+    const double kl = (double)(ps[0] / (double)(KURA_N)) * lam;
+    sbar[0] = sbar[0] + kl * phi[1];
+    sbar[1] = sbar[1] - kl * phi[0];
+}
+
+double sode_field_vjp(int i, double t, double yi, double ps[], double po[], double phi[], double sum[], double sbar[],
+                      double lam)
+{
+    const double kl = (double)(ps[0] / (double)(KURA_N)) * lam;
+    return phi[1] * (sbar[0] - kl * sum[1]) - phi[0] * (sbar[1] + kl * sum[0]);
+}
+
+void sode_field_vjp_params(int i, double t, double yi, double ps[], double po[], double phi[], double sum[],
+                           double lam, double gs[], double go[])
+{
+    gs[0] = gs[0] + lam * ((sum[0] * phi[1] - sum[1] * phi[0]) / (double)(KURA_N));
+    go[0] = go[0] + lam;
 }
 #endif
