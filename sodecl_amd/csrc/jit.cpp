@@ -22,7 +22,7 @@
 #include <fstream>
 #include <sstream>
 #include <mutex>
-#include <regex>
+#include <set>
 
 #include "sodecl_internal.hpp"
 
@@ -61,12 +61,24 @@ std::string strip_comments(const std::string& s)
 
 PluginFeatures detect_features(const std::string& source)
 {
+    // every identifier followed by '(' (a definition, declaration or call), in
+    // one pass (a regular expression per entry point cost 1.2 ms per context)
     const std::string s = strip_comments(source);
-    auto defines = [&](const char* name) {
-        // a function definition or declaration: name '(' ... at file scope
-        std::regex re(std::string("(^|[^A-Za-z0-9_])") + name + "\\s*\\(");
-        return std::regex_search(s, re);
-    };
+    std::set<std::string> called;
+    auto word = [](char ch) { return std::isalnum((unsigned char)ch) || ch == '_'; };
+    for (size_t i = 0; i < s.size();) {
+        if (!word(s[i])) {
+            ++i;
+            continue;
+        }
+        size_t j = i;
+        while (j < s.size() && word(s[j])) ++j;
+        size_t k = j;
+        while (k < s.size() && std::isspace((unsigned char)s[k])) ++k;
+        if (k < s.size() && s[k] == '(') called.insert(s.substr(i, j - i));
+        i = j;
+    }
+    auto defines = [&](const char* name) { return called.count(name) > 0; };
     PluginFeatures f;
     f.sode_system = defines("sode_system");
     f.sode_system_stoch = defines("sode_system_stoch");
