@@ -29,10 +29,11 @@ struct sodecl_batch {
     std::vector<int> cls, steps, order;
     std::vector<long long> yoff, ooff;
     size_t state_size = 0, output_size = 0;
-    // per class: its work items (four orbit slots each, -1: none, longest
+    // per class: its work items (an orbit per slot of its wavefront, -1: none, longest
     // first; one workgroup each), its kernel, LDS size and stream; classes
     // are launched in order of their total cost, the most expensive first
     struct Class {
+        BatchShape shape;
         std::vector<int> items;
         int nitems = 0;
         double cost = 0.0;
@@ -110,6 +111,61 @@ ProgramKey batch_key(const sodecl_batch* b)
     return k;
 }
 
+// Least power of two of lanes that hold neq rows, rows of them on each.
+int lanes_for(int neq, int rows)
+{
+    int lanes = 1;
+    while (lanes * rows < neq) lanes *= 2;
+    return lanes;
+}
+
+// Lanes per orbit and form of every size class.
+//
+// Windowed form (up to 512 equations): eight rows per lane when the whole
+// batch then has at least four wavefronts per SIMD, where instructions count
+// (32768 orbits of 32, 128 and 512 equations: 8.5 ms, against 9.1 ms with four
+// and 9.5 ms with two rows where the class allows it); smaller batches, whose
+// time is the longest orbit's chain of Newton iterations, spread each orbit over
+// more lanes, two rows each (450 orbits of 10, 74 and 200 equations: 0.43
+// against 0.60 ms).  The two cross between 8000 and 16000 orbits of 22 to 512
+// equations (3.4 and 6.8 wavefronts per SIMD).  A power of two of rows keeps the
+// parity of a row's index known to the compiler.
+//
+// Through LDS: 16 lanes up to 32 equations, 32 up to 128, else 64; the
+// 128-equation class ran 2.5-3% faster on 32 lanes (four rows per lane, four
+// wavefronts per SIMD) than on 16 (eight rows, two wavefronts per SIMD by
+// registers), and up to eight rows on 64 lanes fit 168 registers (three
+// wavefronts per SIMD).
+std::vector<BatchShape> batch_shapes(const sodecl_batch* b)
+{
+    int cus = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, b->device) != hipSuccess || cus <= 0)
+        cus = 256;
+    double waves = 0.0;
+    for (int c : b->cls)
+        if (c >= 0 && c < (int)b->class_neq.size()) waves += lanes_for(b->class_neq[c], 8) / 64.0;
+    const bool large = b->cls.empty() || waves >= 4.0 * 4 * cus;
+    std::vector<BatchShape> shapes;
+    for (int neq : b->class_neq) {
+        BatchShape s;
+        s.neq = neq;
+        const int reach = b->features.window_reach;   // 0: no windowed form
+        s.window = reach >= 1 && reach <= 8 && lanes_for(neq, 8) <= 64;
+        if (s.window) {
+            s.rows = large ? 8 : 2;
+            while (s.rows < reach || lanes_for(neq, s.rows) > 64) s.rows *= 2;
+            s.lanes = lanes_for(neq, s.rows);
+            s.waves = 4;
+        } else {
+            s.lanes = neq <= 32 ? 16 : neq <= 128 ? 32 : 64;
+            s.rows = (neq + s.lanes - 1) / s.lanes;
+            s.waves = s.rows <= 2 || (s.lanes == 32 && s.rows <= 4) ? 4 : (s.lanes == 64 && s.rows <= 8) ? 3 : 2;
+        }
+        shapes.push_back(s);
+    }
+    return shapes;
+}
+
 }  // namespace
 
 extern "C" {
@@ -166,7 +222,7 @@ int sodecl_batch_choose_device(sodecl_batch* b, uint32_t device)
 size_t sodecl_batch_compile_only(sodecl_batch* b, const char* arch)
 {
     if (!b) return 0;
-    b->program = assemble_batch_program(b->source, batch_key(b), b->features, b->class_neq);
+    b->program = assemble_batch_program(b->source, batch_key(b), b->features, batch_shapes(b));
     std::vector<char> code;
     std::string log;
     if (!compile_program(b->program, arch ? arch : "gfx950", b->opts.fp_contract, code, log)) {
@@ -206,18 +262,20 @@ int sodecl_batch_setup(sodecl_batch* b, int orbits, const int* orbit_class, cons
     b->order.resize(orbits);
     std::iota(b->order.begin(), b->order.end(), 0);
     std::stable_sort(b->order.begin(), b->order.end(), [&](int a, int c) { return cost[a] > cost[c]; });
-    // work items of each class: one orbit, or up to four consecutive orbits
-    // (similar costs) where the class runs 32 or 16 lanes per orbit
+    // work items of each class: as many consecutive orbits (similar costs) as
+    // share a wavefront
     const int nclass = (int)b->class_neq.size();
+    const std::vector<BatchShape> shapes = batch_shapes(b);
     b->classes.assign(nclass, sodecl_batch::Class{});
+    for (int ci = 0; ci < nclass; ++ci) b->classes[ci].shape = shapes[ci];
     for (int o : b->order) {
         auto& c = b->classes[b->cls[o]];
-        const int opw = 64 / batch_lanes_per_orbit(b->class_neq[b->cls[o]]);
-        if (c.nitems == 0 || c.items[4 * (c.nitems - 1) + opw - 1] >= 0) {
-            c.items.insert(c.items.end(), {-1, -1, -1, -1});
+        const int opw = c.shape.slots();
+        if (c.nitems == 0 || c.items[(size_t)opw * c.nitems - 1] >= 0) {
+            c.items.insert(c.items.end(), opw, -1);
             ++c.nitems;
         }
-        int* slot = &c.items[4 * (c.nitems - 1)];
+        int* slot = &c.items[(size_t)opw * (c.nitems - 1)];
         int k = 0;
         while (slot[k] >= 0) ++k;
         slot[k] = o;
@@ -229,7 +287,7 @@ int sodecl_batch_setup(sodecl_batch* b, int orbits, const int* orbit_class, cons
                      [&](int x, int y) { return b->classes[x].cost > b->classes[y].cost; });
 
     if (!bhip(b, hipSetDevice(b->device), "hipSetDevice")) return 0;
-    b->program = assemble_batch_program(b->source, batch_key(b), b->features, b->class_neq);
+    b->program = assemble_batch_program(b->source, batch_key(b), b->features, shapes);
     std::string log;
     if (!compile_program(b->program, device_arch(b->device), b->opts.fp_contract, b->code, log))
         return bfail(b, "Failed to build program executable:\n" + log);
@@ -242,16 +300,14 @@ int sodecl_batch_setup(sodecl_batch* b, int orbits, const int* orbit_class, cons
         auto& c = b->classes[ci];
         const std::string name = "sodecl_batch_" + std::to_string(ci);
         if (!bhip(b, hipModuleGetFunction(&c.fn, b->module, name.c_str()), "class kernel")) return 0;
-        // LDS per wavefront: per orbit four rows of the class's size (the
-        // evaluation point shared with the right-hand side, three band
-        // rows) and (more than 8) parameters, times the orbits per
-        // wavefront (batch_class.hip)
-        const long n = b->class_neq[ci];
-        const long lpo = batch_lanes_per_orbit((int)n);
-        const long br = (n + lpo - 1) / lpo;
-        const long tlen = br >= 2 ? (n + 15) / 16 * 16 : n;
-        const long per_orbit = 4 * tlen + (b->npar <= 8 ? 0 : b->npar);
-        c.lds_bytes = (size_t)(per_orbit * (64 / lpo)) * sizeof(double);
+        // LDS per wavefront: per orbit (more than 8) parameters, and in the
+        // form through LDS four rows of the class's size (the evaluation point
+        // shared with the right-hand side, three band rows), times the
+        // orbits per wavefront (batch_class.hip)
+        const long n = c.shape.neq;
+        const long tlen = c.shape.rows >= 2 ? (n + 15) / 16 * 16 : n;
+        const long per_orbit = (c.shape.window ? 0 : 4 * tlen) + (b->npar <= 8 ? 0 : b->npar);
+        c.lds_bytes = (size_t)(per_orbit * c.shape.slots()) * sizeof(double);
         if (c.nitems > 0 &&
             !up((void**)&c.d_items, c.items.data(), c.items.size() * sizeof(int), "work items"))
             return 0;

@@ -1,30 +1,38 @@
 // Per-size-class part of the batched implicit integrator.  The host emits
 // this text once per system size class, inside a namespace, after defining
-// _numeq_ and SODECL_LPO (lanes per orbit: 16 for classes of at most 32
-// equations, four orbits per wavefront; 32 up to 128 equations, two orbits;
-// else 64) for that class and including the system plugin there.
+// _numeq_, SODECL_LPO (lanes per orbit, a power of two; 64 / SODECL_LPO orbits
+// share a wavefront) and SODECL_BR (rows per lane) for that class and including the system plugin
+// there.
 //
-// One orbit is integrated by SODECL_LPO lanes of a wavefront:
-//   * components are owned strided (comp = lane + LPO c) for the right-hand
-//     side, the band Jacobian and the Newton update;
-//   * the tridiagonal solve of each Newton iteration runs in parallel over
-//     contiguous row partitions (lane k owns rows [kR, kR + R)): elimination
-//     inside each partition expresses its rows through the last unknown of
-//     the previous partition and its own last unknown, the resulting
-//     tridiagonal system in those LPO unknowns is solved by parallel cyclic
-//     reduction across lanes, and the partition rows follow by substitution.
+// One orbit is integrated by SODECL_LPO lanes of a wavefront.  Two forms:
+//   * windowed (SODECL_WINDOW): the plugin evaluates component i from its
+//     neighbours up to SODE_REACH away (sode_system_window,
+//     calc_jacobian_band_window).  A lane owns SODECL_BR consecutive
+//     components, and the state, residual, band and solve stay in its
+//     registers; only the SODE_REACH outermost components at either end move
+//     to the neighbouring lanes (DPP wavefront shifts).  No LDS, and what the
+//     plugin gives as constant zeros in the band drops out at compile time.
+//   * through LDS, for any component function: components are owned strided
+//     (comp = lane + LPO c) for the right-hand side, the band Jacobian and the
+//     Newton update, and the solve reads its rows back from LDS.
+// In both, the tridiagonal solve of each Newton iteration runs in parallel over
+// contiguous row partitions (lane k owns rows [kR, kR + R)): elimination
+// inside each partition expresses its rows through the last unknown of the
+// previous partition and its own last unknown, the resulting tridiagonal
+// system in those LPO unknowns is solved by parallel cyclic reduction across
+// lanes, and the partition rows follow by substitution.
 // The matrix is the one the reference's tridiagonal sweep solves
 // (ie.cl:10-48, im.cl:3-41): sub-diagonal a_i = J[i][i+1] for i < N-2 (0
 // otherwise), diagonal J[i][i], super-diagonal c_i = J[i+1][i] (c_{N-1} = 0),
 // each entry already scaled to I + s*dt*J.  Solving it by partitions instead
 // of one sweep changes only the rounding.
 
-#define SODECL_BR ((_numeq_ + SODECL_LPO - 1) / SODECL_LPO)   // rows per partition == components per lane
 #define SODECL_OPW (SODECL_BG / SODECL_LPO)                   // orbits per wavefront
-// Every lane owns exactly SODECL_BR components / rows (neq a multiple of
-// LPO): the bounds tests below are then compile-time true.
-#define SODECL_FULL ((_numeq_ % SODECL_LPO) == 0)
+// Every lane owns exactly SODECL_BR components / rows: the bounds tests below are then compile-time true.
+#define SODECL_FULL (_numeq_ == SODECL_LPO * SODECL_BR)
 #define SODECL_OWNS(comp) (SODECL_FULL || (comp) < _numeq_)
+// Row c of this lane's partition exists.
+#define SODECL_ROW(c) (SODECL_FULL || r0 + (c) < _numeq_)
 // LDS index of row i in the solve's arrays.  A 64-bit LDS access serves 16
 // lanes per pass over 32 four-byte banks, so 16 doubles that differ modulo
 // 16 are conflict-free.  The lanes of the solve read row j of their own
@@ -39,19 +47,13 @@
 #define SODECL_TI(i) (i)
 #define SODECL_TLEN (_numeq_)
 #endif
-// LDS doubles per orbit: four rows -- the evaluation point, which the
+// LDS doubles per orbit (the form through LDS): four rows -- the evaluation point, which the
 // right-hand side of the solve (then its solution) overwrites once the
 // Jacobian has read it, and the three band rows -- and the parameters when
 // there are more than 8 (fewer stay in registers).  16 KiB for 512
 // equations, so that ten wavefronts fit a CU's LDS.
 #define SODECL_PLDS (_numpar_ <= 8 ? 0 : _numpar_)
 #define SODECL_ORBIT_LDS (4 * SODECL_TLEN + SODECL_PLDS)
-
-// Coefficients of row i of the reference's tridiagonal matrix.  The band
-// rows are written with the reference's zeros in place (a_i = 0 outside
-// 1 <= i < N-2, c_{N-1} = 0), so reading them needs no test.
-SODECL_INLINE double sodecl_tri_a(const double* up, int i) { return up[SODECL_TI(i)]; }
-SODECL_INLINE double sodecl_tri_c(const double* lo, int i) { return lo[SODECL_TI(i)]; }
 
 // 1/b from the hardware reciprocal and two Newton-Raphson steps (within an
 // ulp); this solve is not the reference's sweep, so only rounding changes.
@@ -80,22 +82,23 @@ SODECL_INLINE void sodecl_pcr_pair32(double v, int lane, double& up, double& dow
 
 // v of orbit lane - s (up) or lane + s (down), 0 past either end of the
 // orbit's lanes.  Orbits of 16 lanes are DPP rows: row shifts, which bring
-// 0 past either end by themselves.  Otherwise distances of one and two are
-// DPP wavefront shifts (with a whole wavefront per orbit the shift brings 0
-// past either end; 32-lane orbits drop what crossed over from the
-// neighbouring orbit), longer ones a bpermute.
+// 0 past either end by themselves (smaller orbits drop what crossed over
+// from the neighbouring one).  Otherwise distances of one and two are DPP
+// wavefront shifts (with a whole wavefront per orbit the shift brings 0 past
+// either end; 32-lane orbits drop what crossed over), longer ones a bpermute.
 SODECL_INLINE double sodecl_pcr_neighbour(double v, int lane, int s, bool up)
 {
-#if SODECL_LPO == 16
-    (void)lane;
-    switch (s) {
-    case 1: return up ? sodecl_dpp<SODECL_DPP_ROW_SHR(1)>(v) : sodecl_dpp<SODECL_DPP_ROW_SHL(1)>(v);
-    case 2: return up ? sodecl_dpp<SODECL_DPP_ROW_SHR(2)>(v) : sodecl_dpp<SODECL_DPP_ROW_SHL(2)>(v);
-    case 4: return up ? sodecl_dpp<SODECL_DPP_ROW_SHR(4)>(v) : sodecl_dpp<SODECL_DPP_ROW_SHL(4)>(v);
-    default: return up ? sodecl_dpp<SODECL_DPP_ROW_SHR(8)>(v) : sodecl_dpp<SODECL_DPP_ROW_SHL(8)>(v);
-    }
-#else
     const bool inside = up ? lane - s >= 0 : lane + s < SODECL_LPO;
+#if SODECL_LPO <= 16
+    double w;
+    switch (s) {
+    case 1: w = up ? sodecl_dpp<SODECL_DPP_ROW_SHR(1)>(v) : sodecl_dpp<SODECL_DPP_ROW_SHL(1)>(v); break;
+    case 2: w = up ? sodecl_dpp<SODECL_DPP_ROW_SHR(2)>(v) : sodecl_dpp<SODECL_DPP_ROW_SHL(2)>(v); break;
+    case 4: w = up ? sodecl_dpp<SODECL_DPP_ROW_SHR(4)>(v) : sodecl_dpp<SODECL_DPP_ROW_SHL(4)>(v); break;
+    default: w = up ? sodecl_dpp<SODECL_DPP_ROW_SHR(8)>(v) : sodecl_dpp<SODECL_DPP_ROW_SHL(8)>(v); break;
+    }
+    return (SODECL_LPO == 16 || inside) ? w : 0.0;
+#else
     if (s <= 2) {
         double w = up ? sodecl_dpp<SODECL_DPP_WAVE_SHR1>(v) : sodecl_dpp<SODECL_DPP_WAVE_SHL1>(v);
         if (s == 2) w = up ? sodecl_dpp<SODECL_DPP_WAVE_SHR1>(w) : sodecl_dpp<SODECL_DPP_WAVE_SHL1>(w);
@@ -106,21 +109,23 @@ SODECL_INLINE double sodecl_pcr_neighbour(double v, int lane, int s, bool up)
 #endif
 }
 
+// v of the wavefront's previous (up) or next lane: row shifts where orbits lie
+// within 16-lane rows, else wavefront shifts.
+SODECL_INLINE double sodecl_shift(double v, bool up)
+{
+#if SODECL_LPO <= 16
+    return up ? sodecl_dpp<SODECL_DPP_ROW_SHR(1)>(v) : sodecl_dpp<SODECL_DPP_ROW_SHL(1)>(v);
+#else
+    return up ? sodecl_dpp<SODECL_DPP_WAVE_SHR1>(v) : sodecl_dpp<SODECL_DPP_WAVE_SHL1>(v);
+#endif
+}
+
 // Sum over the orbit's lanes, the same value on each of them.
 SODECL_INLINE double sodecl_orbit_sum(double v)
 {
-#if SODECL_LPO == 64
-    return sodecl_group_sum(v);
-#else
-    v += sodecl_dpp<SODECL_DPP_XOR1>(v);
-    v += sodecl_dpp<SODECL_DPP_XOR2>(v);
-    v += sodecl_dpp<SODECL_DPP_HALF_MIRROR>(v);
-    v += sodecl_dpp<SODECL_DPP_MIRROR>(v);
-#if SODECL_LPO == 32
-    v += __shfl_xor(v, 16, SODECL_LPO);
-#endif
-    return v;
-#endif
+    double s[1] = {v};
+    sodecl_lane_sums<SODECL_LPO>(s);
+    return s[0];
 }
 
 // Partitions that hold rows, and the cyclic-reduction levels they need
@@ -129,84 +134,80 @@ SODECL_INLINE double sodecl_orbit_sum(double v)
 #define SODECL_PCR_LEVELS (SODECL_NPART > 32 ? 6 : SODECL_NPART > 16 ? 5 : SODECL_NPART > 8 ? 4 : \
                            SODECL_NPART > 4 ? 3 : SODECL_NPART > 2 ? 2 : SODECL_NPART > 1 ? 1 : 0)
 
-// Solves M x = v for the matrix above; lo, di, up, v, x in LDS (padded
-// layout); x may be v (each lane reads only its own partition's rows of v,
-// all before it writes them); all lanes of the wavefront, lane = the lane's
-// index within its orbit.
-SODECL_INLINE void sodecl_tri_solve(const double* lo, const double* di, const double* up, const double* v, double* x,
-                                    int lane)
+// A value known to be a zero when the kernel is compiled: a coefficient the
+// plugin gives as a constant zero.  Its products drop out of the elimination
+// (they would be zeros added to finite values).
+SODECL_INLINE bool sodecl_zero(double v) { return __builtin_constant_p(v) && v == 0.0; }
+
+// Solves M x = v for the matrix above.  Row j of this lane's partition has the
+// sub-diagonal up(j), diagonal di(j) and super-diagonal lo(j) (functions, so that
+// rows in LDS are read where they are used), with the reference's zeros in place (a_i = 0 outside 1 <= i < N-2, c_{N-1} = 0);
+// rows past the last are identity rows (0, 1, 0) with v = 0, so that every
+// partition is complete.  All lanes of the wavefront, lane = the lane's index
+// within its orbit.
+template <class Lo, class Di, class Up, class V>
+SODECL_INLINE void sodecl_tri_solve(Lo lo, Di di, Up up, V v, double (&x)[SODECL_BR], int lane)
 {
-    const int R = SODECL_BR;
-    const int r0 = lane * R;
-    const bool active = SODECL_FULL || r0 < _numeq_;
-    const int r1 = SODECL_FULL ? r0 + R - 1 : (active ? min(_numeq_, r0 + R) - 1 : r0);
-    const int nin = SODECL_FULL ? R - 1 : (active ? r1 - r0 : 0);   // interior rows r0 .. r1-1
-    double ia[SODECL_BR], be[SODECL_BR], ga[SODECL_BR];   // ia = 1/alpha
-    double e[SODECL_BR], f[SODECL_BR], g[SODECL_BR];
+    const int R = SODECL_BR, I = R > 1 ? R - 1 : 1;   // R - 1 interior rows, then the partition's last
+    double ia[I], be[I], ga[I];   // ia = 1/alpha
+    double e[I], f[I], g[I];
     // forward elimination through the interior, tracking the coupling to
     // x_L = last unknown of the previous partition
 #pragma unroll
-    for (int j = 0; j < SODECL_BR - 1; ++j) {
-        if (j < nin) {
-            const int i = r0 + j;
-            double al;
-            if (j == 0) {
-                al = di[SODECL_TI(i)];
-                be[0] = v[SODECL_TI(i)];
-                ga[0] = sodecl_tri_a(up, i);
-            } else {
-                const double m = sodecl_tri_a(up, i) * ia[j - 1];
-                al = di[SODECL_TI(i)] - m * sodecl_tri_c(lo, i - 1);
-                be[j] = v[SODECL_TI(i)] - m * be[j - 1];
-                ga[j] = -m * ga[j - 1];
-            }
-            ia[j] = sodecl_rcp(al);
+    for (int j = 0; j < R - 1; ++j) {
+        double al = di(j);
+        if (j == 0) {
+            be[0] = v(0);
+            ga[0] = up(0);
+        } else if (sodecl_zero(up(j))) {
+            be[j] = v(j);
+            ga[j] = 0.0;
+        } else {
+            const double m = up(j) * ia[j - 1];
+            if (!sodecl_zero(lo(j - 1))) al = di(j) - m * lo(j - 1);
+            be[j] = v(j) - m * be[j - 1];
+            ga[j] = sodecl_zero(ga[j - 1]) ? 0.0 : -m * ga[j - 1];
         }
+        ia[j] = sodecl_rcp(al);
     }
     // backward: interior x_i = e_i + f_i x_L + g_i x_R, x_R = own last unknown
 #pragma unroll
-    for (int j = SODECL_BR - 2; j >= 0; --j) {
-        if (j < nin) {
-            const int i = r0 + j;
-            const double ci = sodecl_tri_c(lo, i);
-            if (j == nin - 1) {
-                e[j] = be[j] * ia[j];
-                f[j] = -ga[j] * ia[j];
-                g[j] = -ci * ia[j];
-            } else {
-                e[j] = (be[j] - ci * e[j + 1]) * ia[j];
-                f[j] = (-ga[j] - ci * f[j + 1]) * ia[j];
-                g[j] = (-ci * g[j + 1]) * ia[j];
-            }
+    for (int j = R - 2; j >= 0; --j) {
+        const double ci = lo(j);
+        f[j] = sodecl_zero(ga[j]) ? 0.0 : -ga[j] * ia[j];
+        if (j == R - 2) {
+            e[j] = be[j] * ia[j];
+            g[j] = sodecl_zero(ci) ? 0.0 : -ci * ia[j];
+        } else if (sodecl_zero(ci)) {
+            e[j] = be[j] * ia[j];
+            g[j] = 0.0;
+        } else {
+            e[j] = (be[j] - ci * e[j + 1]) * ia[j];
+            if (!sodecl_zero(f[j + 1])) f[j] = (-ga[j] - ci * f[j + 1]) * ia[j];
+            g[j] = sodecl_zero(g[j + 1]) ? 0.0 : (-ci * g[j + 1]) * ia[j];
         }
     }
-    // reduced row of partition k (row r1): A X_{k-1} + B X_k + C X_{k+1} = D
-    const bool has_in = nin > 0;
-    const double e_last = has_in ? e[nin - 1] : 0.0;
-    const double f_last = has_in ? f[nin - 1] : 1.0;   // x_{r1-1} is X_{k-1} itself without interior
-    const double g_last = has_in ? g[nin - 1] : 0.0;
-    // the next partition's first row, through X_k and X_{k+1}
-    const double e_first = has_in ? e[0] : 0.0;
-    const double f_first = has_in ? f[0] : 0.0;
-    const double g_first = has_in ? g[0] : 1.0;   // without interior its first row is its X
-    const double e_nx = sodecl_pcr_neighbour(e_first, lane, 1, false);
-    const double f_nx = sodecl_pcr_neighbour(f_first, lane, 1, false);
-    const double g_nx = sodecl_pcr_neighbour(g_first, lane, 1, false);
-    double A = 0.0, B = 1.0, C = 0.0, D = 0.0;
-    if (active) {
-        const double ar = sodecl_tri_a(up, r1);   // zero for row 0
-        const double cr = sodecl_tri_c(lo, r1);
-        const bool has_next = r1 + 1 < _numeq_;
-        A = ar * f_last;
-        B = di[SODECL_TI(r1)] + ar * g_last + (has_next ? cr * f_nx : 0.0);
-        C = has_next ? cr * g_nx : 0.0;
-        D = v[SODECL_TI(r1)] - ar * e_last - (has_next ? cr * e_nx : 0.0);
+    // reduced row of partition k (its last row): A X_{k-1} + B X_k + C X_{k+1} = D.
+    // Without interior the row before the last is X_{k-1} itself, and a
+    // partition's first row is its X.
+    const double e_last = R > 1 ? e[I - 1] : 0.0, f_last = R > 1 ? f[I - 1] : 1.0, g_last = R > 1 ? g[I - 1] : 0.0;
+    double A = 0.0, B = di(R - 1), C = 0.0, D = v(R - 1);
+    if (!sodecl_zero(up(R - 1))) {
+        A = up(R - 1) * f_last;
+        B = B + up(R - 1) * g_last;
+        D = D - up(R - 1) * e_last;
+    }
+    if (!sodecl_zero(lo(R - 1))) {
+        // the next partition's first row, through X_k and X_{k+1}
+        B = B + lo(R - 1) * sodecl_pcr_neighbour(R > 1 ? f[0] : 0.0, lane, 1, false);
+        C = lo(R - 1) * sodecl_pcr_neighbour(R > 1 ? g[0] : 1.0, lane, 1, false);
+        D = D - lo(R - 1) * sodecl_pcr_neighbour(R > 1 ? e[0] : 0.0, lane, 1, false);
     }
     // When every reduced row is already decoupled (A = C = 0: the partition
     // boundaries fall where the matrix has no coupling, as for a system of
     // 2x2 blocks such as the Brusselator chain under the reference's index
     // mapping), cyclic reduction would leave B and D unchanged: skip it.
-    if (!__all(A == 0.0 && C == 0.0)) {
+    if (!(sodecl_zero(A) && sodecl_zero(C)) && !__all(A == 0.0 && C == 0.0)) {
         // parallel cyclic reduction over the reduced rows.  Each lane shares its
         // row scaled by its pivot's reciprocal (A/B, C/B, D/B), so one
         // reciprocal per lane and level and three values per direction suffice:
@@ -242,12 +243,21 @@ SODECL_INLINE void sodecl_tri_solve(const double* lo, const double* di, const do
     }
     const double X = D * sodecl_rcp(B);
     const double Xm = sodecl_pcr_neighbour(X, lane, 1, true);
-    if (active) {
 #pragma unroll
-        for (int j = 0; j < SODECL_BR - 1; ++j)
-            if (j < nin) x[SODECL_TI(r0 + j)] = e[j] + f[j] * Xm + g[j] * X;
-        x[SODECL_TI(r1)] = X;
+    for (int j = 0; j < R - 1; ++j) {
+        x[j] = e[j];
+        if (!sodecl_zero(f[j])) x[j] = x[j] + f[j] * Xm;
+        if (!sodecl_zero(g[j])) x[j] = x[j] + g[j] * X;
     }
+    x[R - 1] = X;
+}
+
+// The most steps of any orbit of the wavefront, in a scalar register.
+SODECL_INLINE int sodecl_wave_steps(int steps)
+{
+#pragma unroll
+    for (int m = SODECL_LPO; m < 64; m <<= 1) steps = max(steps, __shfl_xor(steps, m));
+    return __builtin_amdgcn_readfirstlane(steps);
 }
 
 // The routine is inlined into its class's kernel (a called function gets
@@ -257,8 +267,7 @@ SODECL_INLINE void sodecl_tri_solve(const double* lo, const double* di, const do
 #ifndef SODECL_BATCH_ITEM_ATTR
 #define SODECL_BATCH_ITEM_ATTR __attribute__((always_inline))
 #endif
-// Integrates the orbits of one work item -- SODECL_OPW orbits (1, 2 or 4),
-// item[k] on the k-th group of SODECL_LPO lanes (item[k] < 0: none) -- for steps[o]
+// Integrates the orbits of one work item -- SODECL_OPW orbits, item[k] on the k-th group of SODECL_LPO lanes (item[k] < 0: none) -- for steps[o]
 // steps of implicit Euler (SODECL_SOLVER 3, ie.cl:50-117) or implicit
 // midpoint (4, im.cl:43-118) with the reference's Newton iteration: stop
 // when the L1 (IE) / L2 (IM) residual norm is below _epsilon1_, at most
@@ -268,6 +277,139 @@ SODECL_INLINE void sodecl_tri_solve(const double* lo, const double* di, const do
 // until its longest orbit is done and iterates until every orbit's Newton
 // iteration has stopped; an orbit that has stopped computes along on its
 // last values without storing them or counting updates.
+#if SODECL_WINDOW
+__device__ SODECL_BATCH_ITEM_ATTR void sodecl_batch_item(const int* __restrict__ item, const int* __restrict__ steps_of,
+                                  const long long* __restrict__ yoff, const long long* __restrict__ ooff,
+                                  const double* __restrict__ y0_all, const double* __restrict__ params_all,
+                                  double* __restrict__ out_all, long long* __restrict__ newton, double* lds)
+{
+    static_assert(SODECL_BR >= SODE_REACH, "a component's neighbours sit on the next lane at most");
+    const int part = threadIdx.x / SODECL_LPO;
+    const int lane = threadIdx.x % SODECL_LPO;
+    const int r0 = lane * SODECL_BR;
+    const int o = item[part];
+    const bool has = o >= 0;
+    const int steps = has ? steps_of[o] : 0;
+    const int smax = sodecl_wave_steps(steps);
+    // parameters in registers when there are few, else in LDS
+#if _numpar_ <= 8
+    (void)lds;
+    double sh_p[_numpar_ > 0 ? _numpar_ : 1];
+#pragma unroll
+    for (int k = 0; k < _numpar_; ++k) sh_p[k] = has ? params_all[(size_t)o * _numpar_ + k] : 0.0;
+#else
+    double* const sh_p = lds + (size_t)part * _numpar_;
+    for (int k = lane; k < _numpar_; k += SODECL_LPO) sh_p[k] = has ? params_all[(size_t)o * _numpar_ + k] : 0.0;
+    sodecl_wave_sync();
+#endif
+    double* const out = has ? out_all + ooff[o] : nullptr;
+    double y[SODECL_BR], gg[SODECL_BR];
+#pragma unroll
+    for (int c = 0; c < SODECL_BR; ++c) {
+        y[c] = 0.0;
+        if (has && SODECL_ROW(c)) {
+            y[c] = y0_all[yoff[o] + r0 + c];
+            out[r0 + c] = y[c];
+        }
+    }
+    double t = 0.0;
+    long long updates = 0;
+#if SODECL_SOLVER == 3
+    const double scale = -1.00;
+#else
+    const double scale = -0.50;
+#endif
+    for (int s = 0; s < smax; ++s) {
+        const bool live = s < steps;
+#pragma unroll
+        for (int c = 0; c < SODECL_BR; ++c) gg[c] = y[c];
+        for (int it = 0; it < SODECL_NEWTON_MAXIT; ++it) {
+            // the evaluation point of this lane's components and SODE_REACH
+            // more on either side
+            double win[SODECL_BR + 2 * SODE_REACH];
+#pragma unroll
+            for (int c = 0; c < SODECL_BR; ++c) {
+#if SODECL_SOLVER == 3
+                win[SODE_REACH + c] = gg[c];
+#else
+                win[SODE_REACH + c] = (y[c] + gg[c]) * 0.5;
+#endif
+            }
+#pragma unroll
+            for (int d = 0; d < SODE_REACH; ++d) {
+                // (what crosses over from another orbit stands for components
+                // that do not exist)
+                win[d] = sodecl_shift(win[SODECL_BR + d], true);
+                win[SODE_REACH + SODECL_BR + d] = sodecl_shift(win[SODE_REACH + d], false);
+            }
+            double r[SODECL_BR], lo[SODECL_BR], di[SODECL_BR], up[SODECL_BR], x[SODECL_BR];
+            double err = 0.0;
+#pragma unroll
+            for (int c = 0; c < SODECL_BR; ++c) {
+                r[c] = 0.0;
+                if (SODECL_ROW(c)) {
+                    const double fv = sode_system_window(r0 + c, t, &win[SODE_REACH + c], sh_p);
+                    r[c] = gg[c] - y[c] - fv * _m_dt_;
+#if SODECL_SOLVER == 3
+                    err = err + fabs(r[c]);
+#else
+                    err = err + r[c] * r[c];
+#endif
+                }
+            }
+            // The band does not depend on the residual norm: evaluated while
+            // the reduction and vote are in flight; not used in the iteration
+            // that ends a step.
+#pragma unroll
+            for (int c = 0; c < SODECL_BR; ++c) {
+                lo[c] = 0.0;
+                di[c] = 1.0;
+                up[c] = 0.0;
+                if (SODECL_ROW(c)) {
+                    double l, d, u;
+                    calc_jacobian_band_window(r0 + c, &win[SODE_REACH + c], sh_p, &l, &d, &u);
+                    // a_i = J[i][i+1] for 1 <= i < N-2, c_i = J[i+1][i] for i < N-1, else 0
+                    if (!sodecl_zero(l)) lo[c] = r0 + c < _numeq_ - 1 ? l * scale * _m_dt_ : 0.0;
+                    if (!sodecl_zero(u)) up[c] = (r0 + c >= 1 && r0 + c < _numeq_ - 2) ? u * scale * _m_dt_ : 0.0;
+                    di[c] = d * scale * _m_dt_ + 1;
+                }
+            }
+            err = sodecl_orbit_sum(err);
+#if SODECL_SOLVER == 3
+            const bool done = !live || err < _epsilon1_;
+#else
+            const bool done = !live || sqrt(err) < _epsilon1_;
+#endif
+            if (__all(done)) break;
+            // A residual that is not a number leaves no component a number
+            // (the reference's sweep carries it through every row).
+            if (__builtin_expect(__builtin_amdgcn_ballot_w64(err != err) != 0, 0)) {
+#pragma unroll
+                for (int c = 0; c < SODECL_BR; ++c) r[c] = err != err ? err : r[c];
+            }
+            sodecl_tri_solve([&](int j) { return lo[j]; }, [&](int j) { return di[j]; }, [&](int j) { return up[j]; },
+                             [&](int j) { return r[j]; }, x, lane);
+            if (!done) {
+#pragma unroll
+                for (int c = 0; c < SODECL_BR; ++c) gg[c] = gg[c] - x[c];
+                ++updates;
+            }
+        }
+        if (live) {
+#pragma unroll
+            for (int c = 0; c < SODECL_BR; ++c) y[c] = gg[c];
+        }
+        t = t + _m_dt_;
+        if (live && (s + 1) % _numsteps_ == 0) {
+            double* o_snap = out + (size_t)((s + 1) / _numsteps_) * _numeq_;
+#pragma unroll
+            for (int c = 0; c < SODECL_BR; ++c)
+                if (SODECL_ROW(c)) o_snap[r0 + c] = y[c];
+        }
+    }
+    if (has && lane == 0) newton[o] = updates;
+}
+#else
 __device__ SODECL_BATCH_ITEM_ATTR void sodecl_batch_item(const int* __restrict__ item, const int* __restrict__ steps_of,
                                   const long long* __restrict__ yoff, const long long* __restrict__ ooff,
                                   const double* __restrict__ y0_all, const double* __restrict__ params_all,
@@ -278,13 +420,7 @@ __device__ SODECL_BATCH_ITEM_ATTR void sodecl_batch_item(const int* __restrict__
     const int o = item[part];
     const bool has = o >= 0;
     const int steps = has ? steps_of[o] : 0;
-    int smax = steps;
-#if SODECL_OPW >= 2
-    smax = max(__builtin_amdgcn_readlane(steps, 0), __builtin_amdgcn_readlane(steps, SODECL_LPO));
-#endif
-#if SODECL_OPW == 4
-    smax = max(smax, max(__builtin_amdgcn_readlane(steps, 2 * SODECL_LPO), __builtin_amdgcn_readlane(steps, 3 * SODECL_LPO)));
-#endif
+    const int smax = sodecl_wave_steps(steps);
     double* const sh_g = lds + (size_t)part * SODECL_ORBIT_LDS;   // evaluation point (g, or (y+g)/2), plain layout
     double* const sh_r = sh_g;   // then the residual -> right-hand side -> solution (rotated layout)
     double* const sh_lo = sh_r + SODECL_TLEN;
@@ -384,7 +520,20 @@ __device__ SODECL_BATCH_ITEM_ATTR void sodecl_batch_item(const int* __restrict__
 #endif
             if (__all(done)) break;
             sodecl_wave_sync();
-            sodecl_tri_solve(sh_lo, sh_di, sh_up, sh_r, sh_r, lane);
+            {
+                // this lane's partition, the solution written back in place
+                double px[SODECL_BR];
+                const int r0 = lane * SODECL_BR;
+                auto row = [&](const double* a, int j, double past) {
+                    return SODECL_FULL || r0 + j < _numeq_ ? a[SODECL_TI(r0 + j)] : past;
+                };
+                sodecl_tri_solve([&](int j) { return row(sh_lo, j, 0.0); }, [&](int j) { return row(sh_di, j, 1.0); },
+                                 [&](int j) { return row(sh_up, j, 0.0); }, [&](int j) { return row(sh_r, j, 0.0); }, px,
+                                 lane);
+#pragma unroll
+                for (int j = 0; j < SODECL_BR; ++j)
+                    if (SODECL_FULL || r0 + j < _numeq_) sh_r[SODECL_TI(r0 + j)] = px[j];
+            }
             sodecl_wave_sync();
             if (!done) {
 #pragma unroll
@@ -411,8 +560,8 @@ __device__ SODECL_BATCH_ITEM_ATTR void sodecl_batch_item(const int* __restrict__
     }
     if (has && lane == 0) newton[o] = updates;
 }
+#endif  // SODECL_WINDOW
 
-#undef SODECL_BR
 #undef SODECL_OPW
 #undef SODECL_PLDS
 #undef SODECL_ORBIT_LDS
@@ -422,3 +571,4 @@ __device__ SODECL_BATCH_ITEM_ATTR void sodecl_batch_item(const int* __restrict__
 #undef SODECL_PCR_LEVELS
 #undef SODECL_FULL
 #undef SODECL_OWNS
+#undef SODECL_ROW

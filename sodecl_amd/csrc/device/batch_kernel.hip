@@ -5,12 +5,11 @@
 // of the class's list, which the host orders longest first from neq * steps:
 // the dispatcher starts workgroups in index order as room frees up, so the
 // costliest items start first, and the classes' kernels, launched side by
-// side, share the GPU as their workgroups come and go.  An item holds one
-// orbit, or up to 64 / lanes-per-orbit orbits when the class runs 32 or 16
-// lanes per orbit.  A kernel per class gives each class its own register
+// side, share the GPU as their workgroups come and go.  An item holds
+// SODECL_BATCH_SLOTS orbits, 64 / lanes-per-orbit of the class.  A kernel per class gives each class its own register
 // allocation and occupancy.
 //
-// Packed layouts: items[4 * item + k] = orbit or -1; the initial state of
+// Packed layouts: items[SODECL_BATCH_SLOTS * item + k] = orbit or -1; the initial state of
 // orbit o at y0[yoff[o] .. + neq_o]; its snapshots [snap][neq_o] at
 // out[ooff[o] ...], steps[o] / ksteps + 1 of them; params[orbits][npar];
 // newton[o] receives the Newton updates taken.
@@ -24,5 +23,5 @@ SODECL_BATCH_KERNEL(const int* __restrict__ items, const int* __restrict__ steps
 {
     SODECL_EXP_TABLE_INIT();
     extern __shared__ double sodecl_lds[];
-    SODECL_BATCH_ITEM(items + (size_t)blockIdx.x * 4, steps, yoff, ooff, y0, params, out, newton, sodecl_lds);
+    SODECL_BATCH_ITEM(items + (size_t)blockIdx.x * SODECL_BATCH_SLOTS, steps, yoff, ooff, y0, params, out, newton, sodecl_lds);
 }

@@ -87,6 +87,11 @@ PluginFeatures detect_features(const std::string& source)
     f.stoch_component = defines("sode_system_stoch_i");
     f.jacobian_band = defines("calc_jacobian_band");
     f.jacobian_band_i = defines("calc_jacobian_band_i");
+    if (defines("sode_system_window") && defines("calc_jacobian_band_window")) {
+        const std::string key = "#define SODE_REACH ";   // followed by a literal
+        const size_t at = s.find(key);
+        if (at != std::string::npos) f.window_reach = std::atoi(s.c_str() + at + key.size());
+    }
     f.vjp_group = defines("sode_system_vjp_group");
     f.pairs = defines("sode_pair") && defines("sode_system_pairsum");
     f.field = defines("sode_field") && defines("sode_system_field") && defines("sode_field_own_param");
@@ -260,7 +265,7 @@ std::string assemble_host_program(const std::string& system_source, const Progra
 }
 
 std::string assemble_batch_program(const std::string& system_source, const ProgramKey& k, const PluginFeatures& f,
-                                   const std::vector<int>& class_neq)
+                                   const std::vector<BatchShape>& classes)
 {
     std::ostringstream o;
     o << "// SODECL batched program assembled for hipRTC\n";
@@ -288,22 +293,25 @@ std::string assemble_batch_program(const std::string& system_source, const Progr
     o << "#ifndef M_PI\n#define M_PI 3.14159265358979323846\n#endif\n";
     o << kPreludeSource << "\n";
     // one namespace per size class: the plugin and the per-class solver
-    for (size_t c = 0; c < class_neq.size(); ++c) {
+    for (size_t c = 0; c < classes.size(); ++c) {
         o << "namespace sodecl_cls" << c << " {\n";
-        o << "#define _numeq_ " << class_neq[c] << "\n";
-        o << "#define SODECL_LPO " << batch_lanes_per_orbit(class_neq[c]) << "\n";
+        o << "#define _numeq_ " << classes[c].neq << "\n";
+        o << "#define SODECL_LPO " << classes[c].lanes << "\n";
+        o << "#define SODECL_BR " << classes[c].rows << "\n";
+        o << "#define SODECL_WINDOW " << (classes[c].window ? 1 : 0) << "\n";
         o << "#pragma clang force_cuda_host_device begin\n";
         o << system_begin(k) << "#line 1 \"system.cl\"\n" << system_source << "\n" << system_end(k);
         o << "#pragma clang force_cuda_host_device end\n";
         o << kBatchClassSource << "\n";
-        o << "#undef _numeq_\n#undef SODECL_LPO\n";
+        o << "#undef _numeq_\n#undef SODECL_LPO\n#undef SODECL_BR\n#undef SODECL_WINDOW\n";
         o << "}  // namespace sodecl_cls" << c << "\n";
         // the class's own kernel
         o << "#define SODECL_BATCH_KERNEL sodecl_batch_" << c << "\n";
         o << "#define SODECL_BATCH_ITEM sodecl_cls" << c << "::sodecl_batch_item\n";
-        o << "#define SODECL_BATCH_WAVES " << batch_waves_per_simd(class_neq[c]) << "\n";
+        o << "#define SODECL_BATCH_SLOTS " << classes[c].slots() << "\n";
+        o << "#define SODECL_BATCH_WAVES " << classes[c].waves << "\n";
         o << kBatchKernelSource << "\n";
-        o << "#undef SODECL_BATCH_KERNEL\n#undef SODECL_BATCH_ITEM\n#undef SODECL_BATCH_WAVES\n";
+        o << "#undef SODECL_BATCH_KERNEL\n#undef SODECL_BATCH_ITEM\n#undef SODECL_BATCH_WAVES\n#undef SODECL_BATCH_SLOTS\n";
     }
 
     return o.str();

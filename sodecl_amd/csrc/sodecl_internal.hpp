@@ -22,6 +22,8 @@ struct PluginFeatures {
     bool stoch_component = false;   // double sode_system_stoch_i(int, t, y[], p[], noise[])
     bool jacobian_band = false;     // calc_jacobian_band(y, lower, diag, upper, p)
     bool jacobian_band_i = false;   // calc_jacobian_band_i(i, y, p, *lower, *diag, *upper)
+    int window_reach = 0;           // SODE_REACH of a plugin with sode_system_window and
+                                    // calc_jacobian_band_window (batched solver); 0 without them
     bool vjp_group = false;         // sode_system_vjp_group(...) (adjoint, group schedule)
     bool pairs = false;             // sode_pair + sode_system_pairsum (antisymmetric pairwise drift)
     bool field = false;             // sode_field + sode_system_field (coupling through sums over all components)
@@ -35,6 +37,17 @@ struct PluginFeatures {
 
 PluginFeatures detect_features(const std::string& source);
 std::string strip_comments(const std::string& source);
+
+// How the batched integrator runs a size class of neq equations
+// (device/batch_class.hip).
+struct BatchShape {
+    int neq = 1;
+    int lanes = 64;        // lanes of a wavefront per orbit, a power of two
+    bool window = false;   // components in registers, neighbours by lane shifts
+    int rows = 1;          // consecutive rows (and components) per lane
+    int waves = 2;         // wavefronts per SIMD its register budget is sized for
+    int slots() const { return 64 / lanes; }   // orbits per wavefront
+};
 
 // Everything that selects one compiled program.
 struct ProgramKey {
@@ -69,7 +82,7 @@ std::string assemble_host_program(const std::string& system_source, const Progra
 // Program of the batched implicit integrator: the plugin and the per-class
 // solver once per system size in class_neq, then the persistent kernel.
 std::string assemble_batch_program(const std::string& system_source, const ProgramKey& key, const PluginFeatures& f,
-                                   const std::vector<int>& class_neq);
+                                   const std::vector<BatchShape>& classes);
 
 // A compiled and loaded program.
 struct Program {
@@ -87,25 +100,6 @@ struct Program {
 bool compile_program(const std::string& text, const std::string& arch, int fp_contract, std::vector<char>& code,
                      std::string& log, bool ilp_schedule = false);
 std::string device_arch(int device);
-// Lanes of a wavefront per orbit in the batched integrator for a size class
-// of neq equations: 16 (four orbits per wavefront) up to 32 equations, 32
-// (two orbits) up to 128, else 64.  The 128-equation class ran 2.5-3% faster
-// on 32 lanes (four rows per lane, 110 registers, four wavefronts per SIMD)
-// than on 16 (eight rows per lane, two wavefronts per SIMD by registers).
-inline int batch_lanes_per_orbit(int neq) { return neq <= 32 ? 16 : neq <= 128 ? 32 : 64; }
-// Occupancy hint of a size class's kernel (the wavefronts per SIMD its
-// register budget is sized for): up to two rows per lane, or four rows on
-// 32 lanes, need few registers (four); a whole wavefront per orbit with up
-// to 8 rows per lane fits 168 registers with no spill in its Newton loop
-// (three); otherwise two.
-inline int batch_waves_per_simd(int neq)
-{
-    const int lpo = batch_lanes_per_orbit(neq), rows = (neq + lpo - 1) / lpo;
-    if (rows <= 2) return 4;
-    if (lpo == 32 && rows <= 4) return 4;
-    return (lpo == 64 && rows <= 8) ? 3 : 2;
-}
-
 long num_launches(double tspan, double dt, int ksteps);
 
 }  // namespace sodecl_amd
