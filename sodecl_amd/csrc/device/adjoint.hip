@@ -208,10 +208,14 @@ sodecl_group_adjoint(const double* __restrict__ ckpt_t, const double* __restrict
 // gives mu = A^-T lam and
 //   dL/dy += mu                     (IE)   mu + (dt/2) J^T mu   (IM)
 //   dL/dp += dt (df/dp)^T mu        at g (IE) or m (IM).
-// A^T mu = lam is solved like the forward Newton system, by sweeps of a
-// tridiagonal (Thomas) solve: mu += T^-1 (lam - A^T mu) with T the
-// tridiagonal band of A^T, until the residual's L1 norm is below 1e-15 of
-// lam's or after SODECL_NEWTON_MAXIT sweeps.  (The forward's sweep keeps the
+// A^T mu = lam is solved by refinement with an approximate inverse,
+// mu += T^-1 (lam - A^T mu), until the residual's L1 norm is below 1e-15 of
+// lam's or after SODECL_NEWTON_MAXIT rounds.  Up to 12 equations T is A^T
+// itself, eliminated once per step (no pivoting: A is the identity and a
+// multiple of dt), whose rounds end after one or two; constant zeros of the
+// plugin's Jacobian drop out at compile time.  Beyond, T is the tridiagonal
+// band of A^T, as in the forward Newton system (one round costs N^2 instead
+// of N^3 operations).  (The forward's sweep keeps the
 // reference's index quirks because its iterates must match the reference;
 // the adjoint has no reference counterpart and uses the band of A^T as it
 // is.)  For a tridiagonal J one sweep is exact.
@@ -222,14 +226,61 @@ sodecl_group_adjoint(const double* __restrict__ ckpt_t, const double* __restrict
 // entry without its sign), and calc_jacobian_params(y, jp[neq][npar], p)
 // (df/dp).  Checkpoint
 // segments are recomputed with the forward Newton step; the states of a
-// segment go to the workspace laid out [row][neq + 1][orbits] (state and t
-// of row k = step sb + k, rows 0..ckpt_every), orbit-contiguous so the
-// lanes' accesses coalesce.
+// segment go to the workspace laid out [row][neq + 1][orbits] (row k: the
+// state before step sb + k), orbit-contiguous so the lanes' accesses coalesce.
 // ---------------------------------------------------------------------------
 #if SODECL_SCHEDULE == 1 && defined(SODECL_ADJOINT) && SODECL_IS_IMPLICIT && SODECL_HAS_JACOBIAN && \
     SODECL_HAS_JACOBIAN_PARAMS
 
+#if _numpar_ <= 32
+#define SODECL_UNROLL_PARAMS _Pragma("unroll")
+#else
+#define SODECL_UNROLL_PARAMS
+#endif
 #define SODECL_IMPLICIT_C (SODECL_SOLVER == 3 ? 1.0 : 0.50)
+
+// LU elimination of A^T in place of the tridiagonal band
+#define SODECL_ADJOINT_LU (_numeq_ <= 12)
+#if SODECL_ADJOINT_LU
+// lu = A^T = I - cdt J^T on entry; on return its factors (unit lower part
+// below the diagonal), the diagonal as reciprocals.
+SODECL_INLINE void sodecl_lu(double (&lu)[_numeq_][_numeq_])
+{
+#pragma unroll
+    for (int k = 0; k < _numeq_; ++k) {
+        lu[k][k] = sodecl_recip(lu[k][k]);
+#pragma unroll
+        for (int i = k + 1; i < _numeq_; ++i) {
+            if (sodecl_zero(lu[i][k])) continue;
+            lu[i][k] = lu[i][k] * lu[k][k];
+#pragma unroll
+            for (int j = k + 1; j < _numeq_; ++j) {
+                if (sodecl_zero(lu[k][j])) continue;
+                const double q = lu[i][k] * lu[k][j];
+                lu[i][j] = sodecl_zero(lu[i][j]) ? -q : lu[i][j] - q;
+            }
+        }
+    }
+}
+
+SODECL_INLINE void sodecl_lu_solve(const double (&lu)[_numeq_][_numeq_], const double* rhs, double* x)
+{
+#pragma unroll
+    for (int i = 0; i < _numeq_; ++i) {
+        x[i] = rhs[i];
+#pragma unroll
+        for (int k = 0; k < i; ++k)
+            if (!sodecl_zero(lu[i][k])) x[i] = x[i] - lu[i][k] * x[k];
+    }
+#pragma unroll
+    for (int i = _numeq_ - 1; i >= 0; --i) {
+#pragma unroll
+        for (int k = i + 1; k < _numeq_; ++k)
+            if (!sodecl_zero(lu[i][k])) x[i] = x[i] - lu[i][k] * x[k];
+        x[i] = x[i] * lu[i][i];
+    }
+}
+#endif
 
 // Tridiagonal solve (Thomas): row m is sub[m] x[m-1] + dia[m] x[m] +
 // sup[m] x[m+1] = rhs[m].
@@ -261,6 +312,7 @@ sodecl_lane_adjoint(const double* __restrict__ ckpt_t, const double* __restrict_
     const int i = blockIdx.x * SODECL_BLOCK + threadIdx.x;
     if (i >= orbits) return;
     double p[SODECL_NPAR_ALLOC], gp[SODECL_NPAR_ALLOC];
+    SODECL_UNROLL_PARAMS
     for (int m = 0; m < _numpar_; ++m) {
         p[m] = params[(size_t)i * _numpar_ + m];
         gp[m] = 0.0;
@@ -282,29 +334,37 @@ sodecl_lane_adjoint(const double* __restrict__ ckpt_t, const double* __restrict_
         for (int m = 0; m < _numeq_; ++m) y[m] = ckpt_y[(size_t)seg * slab + (size_t)m * orbits + i];
         double t = ckpt_t[(size_t)seg * orbits + i];
         // forward recompute of the segment with the forward Newton step
-        for (int s = sb; s <= se; ++s) {
+        for (int s = sb; s < se; ++s) {
             double* row = work + (size_t)(s - sb) * wrow + i;
             SODECL_UNROLL
             for (int m = 0; m < _numeq_; ++m) row[(size_t)m * orbits] = y[m];
-            row[(size_t)_numeq_ * orbits] = t;
-            if (s == se) break;
             sodecl_implicit_step(t, y, g, p);
             SODECL_UNROLL
             for (int m = 0; m < _numeq_; ++m) y[m] = g[m];
             t = t + _m_dt_;
         }
-        // backward sweep
+        // backward sweep: y is the state after step s (at first the segment's
+        // last, from the recomputation), the state before it was loaded a step
+        // ahead (a launch of few wavefronts has no other to wait for the load)
+        double before[_numeq_];
+        SODECL_UNROLL
+        for (int m = 0; m < _numeq_; ++m)
+            before[m] = work[(size_t)(se - 1 - sb) * wrow + (size_t)m * orbits + i];
         for (int s = se - 1; s >= sb; --s) {
-            const double* r0 = work + (size_t)(s - sb) * wrow + i;
-            const double* r1 = r0 + wrow;
             double x[_numeq_];   // point of J and df/dp: g (IE) or (y + g) / 2 (IM)
             SODECL_UNROLL
             for (int m = 0; m < _numeq_; ++m) {
 #if SODECL_SOLVER == 3
-                x[m] = r1[(size_t)m * orbits];
+                x[m] = y[m];
 #else
-                x[m] = (r0[(size_t)m * orbits] + r1[(size_t)m * orbits]) * 0.5;
+                x[m] = (before[m] + y[m]) * 0.5;
 #endif
+                y[m] = before[m];
+            }
+            if (s > sb) {
+                const double* row = work + (size_t)(s - 1 - sb) * wrow + i;
+                SODECL_UNROLL
+                for (int m = 0; m < _numeq_; ++m) before[m] = row[(size_t)m * orbits];
             }
             double jac[_numeq_][_numeq_];
 #if SODECL_HAS_JACOBIAN_EXACT
@@ -314,6 +374,15 @@ sodecl_lane_adjoint(const double* __restrict__ ckpt_t, const double* __restrict_
 #endif
             // tridiagonal band of A^T: A^T[m][m-1] = A[m-1][m], A^T[m][m+1] = A[m+1][m]
             const double cdt = SODECL_IMPLICIT_C * _m_dt_;
+#if SODECL_ADJOINT_LU
+            double lu[_numeq_][_numeq_];
+#pragma unroll
+            for (int m = 0; m < _numeq_; ++m)
+#pragma unroll
+                for (int k = 0; k < _numeq_; ++k)
+                    lu[m][k] = sodecl_zero(jac[k][m]) ? (m == k ? 1.0 : 0.0) : (m == k ? 1.0 : 0.0) - cdt * jac[k][m];
+            sodecl_lu(lu);
+#else
             double tsub[_numeq_], di[_numeq_], tsup[_numeq_];
             SODECL_UNROLL
             for (int m = 0; m < _numeq_; ++m) {
@@ -321,6 +390,7 @@ sodecl_lane_adjoint(const double* __restrict__ ckpt_t, const double* __restrict_
                 tsub[m] = m > 0 ? -cdt * jac[m - 1][m] : 0.0;
                 tsup[m] = m + 1 < _numeq_ ? -cdt * jac[m + 1][m] : 0.0;
             }
+#endif
             // A^T mu = lam, A = I - c dt J
             double mu[_numeq_], res[_numeq_], d[_numeq_];
             double lnorm = 0.0;
@@ -335,7 +405,11 @@ sodecl_lane_adjoint(const double* __restrict__ ckpt_t, const double* __restrict_
                 SODECL_UNROLL
                 for (int m = 0; m < _numeq_; ++m) rnorm += fabs(res[m]);
                 if (!(rnorm > 1e-15 * lnorm)) break;
+#if SODECL_ADJOINT_LU
+                sodecl_lu_solve(lu, res, d);
+#else
                 sodecl_tridiag(tsub, di, tsup, res, d);
+#endif
                 SODECL_UNROLL
                 for (int m = 0; m < _numeq_; ++m) mu[m] += d[m];
                 // res = lam - A^T mu = lam - mu + c dt J^T mu
@@ -343,7 +417,8 @@ sodecl_lane_adjoint(const double* __restrict__ ckpt_t, const double* __restrict_
                 for (int m = 0; m < _numeq_; ++m) {
                     double a = 0.0;
                     SODECL_UNROLL
-                    for (int k = 0; k < _numeq_; ++k) a += jac[k][m] * mu[k];
+                    for (int k = 0; k < _numeq_; ++k)
+                        if (!sodecl_zero(jac[k][m])) a += jac[k][m] * mu[k];
                     res[m] = lam[m] - mu[m] + cdt * a;
                 }
             }
@@ -351,10 +426,12 @@ sodecl_lane_adjoint(const double* __restrict__ ckpt_t, const double* __restrict_
             if (_numpar_ > 0) {
                 double jp[_numeq_][SODECL_NPAR_ALLOC];
                 calc_jacobian_params(x, jp, p);
+                SODECL_UNROLL_PARAMS
                 for (int k = 0; k < _numpar_; ++k) {
                     double a = 0.0;
                     SODECL_UNROLL
-                    for (int m = 0; m < _numeq_; ++m) a += jp[m][k] * mu[m];
+                    for (int m = 0; m < _numeq_; ++m)
+                        if (!sodecl_zero(jp[m][k])) a += jp[m][k] * mu[m];
                     gp[k] += _m_dt_ * a;
                 }
             }
@@ -366,7 +443,8 @@ sodecl_lane_adjoint(const double* __restrict__ ckpt_t, const double* __restrict_
 #else
                 double a = 0.0;
                 SODECL_UNROLL
-                for (int k = 0; k < _numeq_; ++k) a += jac[k][m] * mu[k];
+                for (int k = 0; k < _numeq_; ++k)
+                    if (!sodecl_zero(jac[k][m])) a += jac[k][m] * mu[k];
                 lam[m] = mu[m] + (0.50 * _m_dt_) * a;
 #endif
             }

@@ -55,16 +55,6 @@
 #define SODECL_PLDS (_numpar_ <= 8 ? 0 : _numpar_)
 #define SODECL_ORBIT_LDS (4 * SODECL_TLEN + SODECL_PLDS)
 
-// 1/b from the hardware reciprocal and two Newton-Raphson steps (within an
-// ulp); this solve is not the reference's sweep, so only rounding changes.
-SODECL_INLINE double sodecl_rcp(double b)
-{
-    double r = __builtin_amdgcn_rcp(b);
-    r = fma(r, fma(-b, r, 1.0), r);
-    r = fma(r, fma(-b, r, 1.0), r);
-    return r;
-}
-
 // The values of lanes l - 32 (up) and l + 32 (down), 0 past either end of
 // the wavefront, from one half-wavefront swap (v_permlane32_swap) per 32-bit
 // half: with both operands v, its first result holds lane l mod 32's value
@@ -133,11 +123,6 @@ SODECL_INLINE double sodecl_orbit_sum(double v)
 #define SODECL_NPART ((_numeq_ + SODECL_BR - 1) / SODECL_BR)
 #define SODECL_PCR_LEVELS (SODECL_NPART > 32 ? 6 : SODECL_NPART > 16 ? 5 : SODECL_NPART > 8 ? 4 : \
                            SODECL_NPART > 4 ? 3 : SODECL_NPART > 2 ? 2 : SODECL_NPART > 1 ? 1 : 0)
-
-// A value known to be a zero when the kernel is compiled: a coefficient the
-// plugin gives as a constant zero.  Its products drop out of the elimination
-// (they would be zeros added to finite values).
-SODECL_INLINE bool sodecl_zero(double v) { return __builtin_constant_p(v) && v == 0.0; }
 
 // Solves M x = v for the matrix above.  Row j of this lane's partition has the
 // sub-diagonal up(j), diagonal di(j) and super-diagonal lo(j) (functions, so that

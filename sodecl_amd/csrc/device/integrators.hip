@@ -111,6 +111,13 @@ SODECL_INLINE void sodecl_noise_pair(int orbit, sodecl_u64 word, double dtsqrt, 
 // ---------------------------------------------------------------------------
 #if SODECL_IS_IMPLICIT
 
+// v * scale * dt; on the GPU a constant zero stays one for the sweep to see.
+#if defined(SODECL_HOST_BUILD)
+#define SODECL_SCALED(v) ((v) * scale * _m_dt_)
+#else
+#define SODECL_SCALED(v) (sodecl_zero(v) ? 0.0 : (v) * scale * _m_dt_)
+#endif
+
 // Three diagonals of I + scale*J at g (ie.cl:83-92, im.cl:84-93: every entry
 // multiplied by scale then by dt, then 1 added to the diagonal).
 SODECL_INLINE void sodecl_newton_band(double* g, double* p, double scale, double* lo, double* di, double* up)
@@ -119,8 +126,8 @@ SODECL_INLINE void sodecl_newton_band(double* g, double* p, double scale, double
     calc_jacobian_band(g, lo, di, up, p);
     SODECL_UNROLL
     for (int i = 0; i < _numeq_; ++i) {
-        lo[i] = lo[i] * scale * _m_dt_;
-        up[i] = up[i] * scale * _m_dt_;
+        lo[i] = SODECL_SCALED(lo[i]);
+        up[i] = SODECL_SCALED(up[i]);
         di[i] = di[i] * scale * _m_dt_;
         di[i] = di[i] + 1;
     }
@@ -131,17 +138,48 @@ SODECL_INLINE void sodecl_newton_band(double* g, double* p, double scale, double
     for (int i = 0; i < _numeq_; ++i) {
         di[i] = jac[i][i] * scale * _m_dt_;
         di[i] = di[i] + 1;
-        up[i] = (i + 1 < _numeq_) ? jac[i][i + 1] * scale * _m_dt_ : 0.0;
-        lo[i] = (i + 1 < _numeq_) ? jac[i + 1][i] * scale * _m_dt_ : 0.0;
+        up[i] = (i + 1 < _numeq_) ? SODECL_SCALED(jac[i][i + 1]) : 0.0;
+        lo[i] = (i + 1 < _numeq_) ? SODECL_SCALED(jac[i + 1][i]) : 0.0;
     }
 #endif
 }
 
+#if !defined(SODECL_HOST_BUILD)
+// 1/b within an ulp, zeros, infinities and NaN as IEEE division gives them.
+SODECL_INLINE double sodecl_recip(double b) { return __builtin_amdgcn_div_fixup(sodecl_rcp(b), b, 1.0); }
+#endif
+
 // The reference's "Thomas" sweep (ie.cl:10-48): a Thomas solve of the
 // tridiagonal matrix with sub-diagonal a[i] = J[i][i+1] (zero for i >= N-2),
 // diagonal b[i] = J[i][i] and super-diagonal c[i] = J[i+1][i]; v is consumed.
+// In the default arithmetic on the GPU each row's two divisions by its pivot
+// become products with one reciprocal (six instructions with its special
+// cases, against eleven and the hardware reciprocal's four issue slots for
+// each division), and coefficients that are constant zeros in the plugin drop
+// out.
 SODECL_INLINE void sodecl_thomas(const double* lo, const double* di, const double* up, double* v, double* x)
 {
+#if !SODECL_STRICT && !defined(SODECL_HOST_BUILD)
+    double rb[_numeq_];
+    rb[0] = sodecl_recip(di[0]);
+    SODECL_UNROLL
+    for (int i = 1; i < _numeq_; ++i) {
+        double b = di[i];
+        if (i < _numeq_ - 2 && !sodecl_zero(up[i])) {
+            const double m = up[i] * rb[i - 1];
+            if (!sodecl_zero(lo[i - 1])) b = di[i] - m * lo[i - 1];
+            v[i] = v[i] - m * v[i - 1];
+        }
+        rb[i] = sodecl_recip(b);
+    }
+    x[_numeq_ - 1] = v[_numeq_ - 1] * rb[_numeq_ - 1];
+    SODECL_UNROLL
+    for (int i = _numeq_ - 2; i >= 0; --i) {
+        double w = v[i];
+        if (!sodecl_zero(lo[i])) w = w - lo[i] * x[i + 1];
+        x[i] = w * rb[i];
+    }
+#else
     double b[_numeq_];
     b[0] = di[0];
     SODECL_UNROLL
@@ -156,6 +194,7 @@ SODECL_INLINE void sodecl_thomas(const double* lo, const double* di, const doubl
     for (int i = _numeq_ - 2; i >= 0; --i) {
         x[i] = (v[i] - lo[i] * x[i + 1]) / b[i];
     }
+#endif
 }
 
 // One implicit step from y: implicit Euler (ie.cl:50-117, L1 stop test,

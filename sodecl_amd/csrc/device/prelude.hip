@@ -22,6 +22,24 @@ __device__ inline double sodecl_dpp(double v)
 #define SODECL_DPP_ROW_SHR(n) (0x110 + (n))   // lane i <- lane i - n within its 16-lane row (0 past the start)
 #define SODECL_DPP_ROW_SHL(n) (0x100 + (n))   // lane i <- lane i + n within its 16-lane row (0 past the end)
 
+// 1/b from the hardware reciprocal and two Newton-Raphson steps (within an
+// ulp, for solves that are not the reference's operation by operation).
+__device__ inline double sodecl_rcp(double b)
+{
+    double r = __builtin_amdgcn_rcp(b);
+    r = fma(r, fma(-b, r, 1.0), r);
+    r = fma(r, fma(-b, r, 1.0), r);
+    return r;
+}
+
+// A value known to be a zero when the kernel is compiled: a coefficient the
+// plugin gives as a constant zero.  Its products drop out of an elimination or
+// a sum (they would be zeros added to finite values).
+__device__ __attribute__((always_inline)) inline bool sodecl_zero(double v)
+{
+    return __builtin_constant_p(v) && v == 0.0;
+}
+
 // Orders this wavefront's LDS accesses before the call against those after
 // it, for exchanges among the lanes of one wavefront: DS instructions of one
 // wavefront execute in order, and the fences plus the wave barrier keep the

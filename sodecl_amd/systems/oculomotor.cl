@@ -59,6 +59,15 @@ double ocu_div(double a, double d, double rd)
 #endif
 }
 
+/* exp(-|x|/bt) and exp(-|x|/b).  In the GPU's default arithmetic every burst
+ * curve and derivative at one point is written with this pair, so that the
+ * compiler evaluates its two exponentials once for all of them. */
+void ocu_exps(double x, double b, double bt, double* es, double* er)
+{
+    *es = exp(ocu_div(-fabs(x), bt, 1.0 / bt));
+    *er = exp(ocu_div(-fabs(x), b, 1.0 / b));
+}
+
 /* Burst-neuron firing curve: saturating exponential for x > 0, a scaled
  * x*exp(x/b) ramp otherwise.  The exponent is selected before the single
  * exp() call, so lanes of a wavefront that take different sides still
@@ -68,6 +77,11 @@ double ocu_div(double a, double d, double rd)
 double ocu_burst(double x, double a, double b, double at, double bt)
 {
     const int pos = x > 0;
+#if defined(SODECL_STRICT) && !SODECL_STRICT && SODECL_SOLVER > 2
+    double es, er;
+    ocu_exps(x, b, bt, &es, &er);
+    return pos ? at * (1.00 - es) : -(a / b) * x * er;
+#else
     /* one division through the selected parameter's reciprocal; both
      * reciprocals depend on the orbit only and are computed once per run.
      * (2/bt)*0.5 is exactly 1/bt (scaling by powers of two commutes with
@@ -80,6 +94,7 @@ double ocu_burst(double x, double a, double b, double at, double bt)
      * modifier; for x = +0 it is -0, whose quotient's exp is 1 as well */
     const double e = exp(ocu_div(-fabs(x), pos ? bt : b, pos ? rbt : rb));
     return pos ? at * (1.00 - e) : -(a / b) * x * e;
+#endif
 }
 
 /* Both burst curves of the right-hand side, B(x) and B(-x), with their
@@ -94,8 +109,10 @@ double ocu_burst(double x, double a, double b, double at, double bt)
  * in sign).  Each result has the bits of ocu_burst's. */
 void ocu_burst_pair(double x, double a, double b, double at, double bt, double* bx, double* bmx)
 {
-    const double sat = at * (1.00 - exp(ocu_div(-fabs(x), bt, 1.0 / bt)));
-    const double ramp = -(a / b) * x * exp(ocu_div(-fabs(x), b, 1.0 / b));
+    double es, er;
+    ocu_exps(x, b, bt, &es, &er);
+    const double sat = at * (1.00 - es);
+    const double ramp = -(a / b) * x * er;
     *bx = x > 0 ? sat : ramp;
     *bmx = x < 0 ? sat : -ramp;
 }
@@ -104,7 +121,13 @@ void ocu_burst_pair(double x, double a, double b, double at, double bt, double* 
 double ocu_burst_dx(double x, double a, double b, double at, double bt)
 {
     const int pos = x > 0;
+#if defined(SODECL_STRICT) && !SODECL_STRICT
+    double es, er;
+    ocu_exps(x, b, bt, &es, &er);
+    const double e = pos ? es : er;
+#else
     const double e = exp((pos ? -x : x) / (pos ? bt : b));
+#endif
     return pos ? (at * e) / bt : -((a * e) / b + (a * x * e) / (b * b));
 }
 
@@ -229,9 +252,11 @@ void calc_jacobian_exact(double y[_numeq_], double jac[_numeq_][_numeq_], double
  * (a, b, at, bt). */
 void ocu_burst_dp(double x, double a, double b, double at, double bt, double d[4])
 {
+    double es, er;
+    ocu_exps(x, b, bt, &es, &er);
     if (x > 0)
     {
-        const double e = exp(-x / bt);
+        const double e = es;
         d[0] = 0;
         d[1] = 0;
         d[2] = 1.00 - e;
@@ -239,7 +264,7 @@ void ocu_burst_dp(double x, double a, double b, double at, double bt, double d[4
     }
     else
     {
-        const double e = exp(x / b);
+        const double e = er;
         d[0] = -(x / b) * e;
         d[1] = ((a * x * e) / (b * b)) * (1.00 + x / b);
         d[2] = 0;
