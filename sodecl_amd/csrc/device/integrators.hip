@@ -308,9 +308,26 @@ SODECL_INLINE int sodecl_lane_step(double t, double* y, double* yout, double* p)
 //   newton: per-orbit Newton update counts (implicit solvers) or null.
 // ---------------------------------------------------------------------------
 #if SODECL_SCHEDULE == 1
-// Orbit i of a lane-schedule launch: one lane of sodecl_lane, or one
-// iteration of the host share's orbit loop (SODECL_HOST_BUILD).
-SODECL_INLINE void sodecl_lane_orbit(int i, double* __restrict__ t_state, double* __restrict__ y_state,
+// Lanes per orbit (1 except for the noise of small Euler-Maruyama launches).
+// The noise does not depend on the state, and drawing it is most of a small
+// system's step (230 of the 356 VALU instructions of the oculomotor model's):
+// where a launch leaves SIMDs idle, SODECL_NL lanes integrate each orbit
+// together, and once every SODECL_NL steps lane j draws the noise of step j
+// ahead (Threefry counters as in sequence) into LDS, from where every lane
+// reads the current step's.  All of them carry the same state with the same
+// bits; lane 0 stores it.
+#ifndef SODECL_NL
+#define SODECL_NL 1
+#endif
+#if SODECL_NL > 1
+// one orbit's noise buffer (odd: orbits of a wavefront read different banks)
+#define SODECL_NOISE_ROW ((SODECL_NL * SODECL_NNOI_ALLOC) | 1)
+#endif
+
+// Orbit i of a lane-schedule launch: one lane of sodecl_lane (lane sub of its
+// SODECL_NL, with the orbit's noise buffer), or one iteration of the host
+// share's orbit loop (SODECL_HOST_BUILD).
+SODECL_INLINE void sodecl_lane_orbit(int i, int sub, double* buffer, double* __restrict__ t_state, double* __restrict__ y_state,
                                      const double* __restrict__ params, double* __restrict__ counters,
                                      double* __restrict__ traj, long long* __restrict__ newton, int orbits, int s0,
                                      int nseg, int final_snap, double* __restrict__ ckpt_t,
@@ -327,14 +344,18 @@ SODECL_INLINE void sodecl_lane_orbit(int i, double* __restrict__ t_state, double
     const double dtsqrt = sqrt(_m_dt_);
     const int calls = (int)ceilf((float)((float)(_numnoi_) * 0.5));
     double noise[SODECL_NNOI_ALLOC];
+#if SODECL_NL > 1
+    int drawn = SODECL_NL;   // step of the buffer that comes next: none left
 #endif
+#endif
+    (void)buffer;
     long long nu = 0;
     // checkpoint k is the state before global step k * ckpt_every
     long long ck = ckpt_y ? (gstep0 + ckpt_every - 1) / ckpt_every : 0;   // next checkpoint index
     long long ck_step = ck * ckpt_every;
     long long g = gstep0;
     for (int s = 0; s < nseg; ++s) {
-        if (traj) {
+        if (traj && sub == 0) {
             double* o = traj + (size_t)(s0 + s) * slab + i;
             SODECL_UNROLL
             for (int m = 0; m < _numeq_; ++m) o[(size_t)m * orbits] = y[m];
@@ -348,9 +369,11 @@ SODECL_INLINE void sodecl_lane_orbit(int i, double* __restrict__ t_state, double
                 if (g == ck_step) {
                     const long long k = ck++;
                     ck_step += ckpt_every;
-                    SODECL_UNROLL
-                    for (int m = 0; m < _numeq_; ++m) ckpt_y[(size_t)k * slab + (size_t)m * orbits + i] = y[m];
-                    ckpt_t[(size_t)k * orbits + i] = t;
+                    if (sub == 0) {
+                        SODECL_UNROLL
+                        for (int m = 0; m < _numeq_; ++m) ckpt_y[(size_t)k * slab + (size_t)m * orbits + i] = y[m];
+                        ckpt_t[(size_t)k * orbits + i] = t;
+                    }
                 }
                 if (ck_step - g < run) run = (int)(ck_step - g);   // g < ck_step here
             }
@@ -359,6 +382,23 @@ SODECL_INLINE void sodecl_lane_orbit(int i, double* __restrict__ t_state, double
             for (; run > 0; --run) {
 #if SODECL_IS_SDE
                 // Noise for this step (stochastic_solver_caller.cl:44-66)
+#if SODECL_NL > 1
+                if (drawn == SODECL_NL) {
+                    sodecl_wave_sync();   // the buffer's last step has been read
+                    const double first = cnt + (double)(sub * SODECL_CALLS);
+                    for (int in = 0; in < SODECL_CALLS; ++in) {
+                        double z0, z1;
+                        sodecl_noise_pair(i, sodecl_counter_word(first + (double)in), dtsqrt, &z0, &z1);
+                        buffer[sub * _numnoi_ + 2 * in] = z0;
+                        if (2 * in + 1 < _numnoi_) buffer[sub * _numnoi_ + 2 * in + 1] = z1;
+                    }
+                    sodecl_wave_sync();
+                    drawn = 0;
+                }
+                for (int in = 0; in < _numnoi_; ++in) noise[in] = buffer[drawn * _numnoi_ + in];
+                ++drawn;
+                cnt = cnt + (double)calls;
+#else
                 int nc = 0;
                 for (int in = 0; in < calls; ++in) {
                     double z0, z1;
@@ -367,6 +407,7 @@ SODECL_INLINE void sodecl_lane_orbit(int i, double* __restrict__ t_state, double
                     if (nc < _numnoi_) noise[nc++] = z0;
                     if (nc < _numnoi_) noise[nc++] = z1;
                 }
+#endif
                 // Euler-Maruyama (stochastic_euler.cl:10-22)
                 {
                     double st[_numeq_];
@@ -384,6 +425,7 @@ SODECL_INLINE void sodecl_lane_orbit(int i, double* __restrict__ t_state, double
             }
         }
     }
+    if (sub != 0) return;
     if (traj && final_snap) {
         double* o = traj + (size_t)(s0 + nseg) * slab + i;
         SODECL_UNROLL
@@ -409,7 +451,7 @@ extern "C" void sodecl_host_lane(double* t_state, double* y_state, const double*
     // of a few orbits per thread must still spread over every thread
 #pragma omp parallel for schedule(dynamic, 1) num_threads(nthreads > 0 ? nthreads : 1)
     for (int i = first; i < last; ++i)
-        sodecl_lane_orbit(i, t_state, y_state, params, counters, traj, newton, orbits, s0, nseg, final_snap, nullptr,
+        sodecl_lane_orbit(i, 0, nullptr, t_state, y_state, params, counters, traj, newton, orbits, s0, nseg, final_snap, nullptr,
                           nullptr, 1, gstep0);
 }
 #else
@@ -421,11 +463,18 @@ sodecl_lane(double* __restrict__ t_state, double* __restrict__ y_state, const do
             long long ws_steps)
 {
     SODECL_EXP_TABLE_INIT();
-    const int i = blockIdx.x * SODECL_BLOCK + threadIdx.x;
+    const int gid = blockIdx.x * SODECL_BLOCK + threadIdx.x;
+    const int i = gid / SODECL_NL;   // an orbit's lanes sit in one wavefront and exit together
     if (i >= orbits) return;
     (void)stage_ws;
     (void)ws_steps;
-    sodecl_lane_orbit(i, t_state, y_state, params, counters, traj, newton, orbits, s0, nseg, final_snap, ckpt_t,
+#if SODECL_NL > 1
+    __shared__ double noise[SODECL_BLOCK / SODECL_NL][SODECL_NOISE_ROW];
+    double* const buffer = noise[threadIdx.x / SODECL_NL];
+#else
+    double* const buffer = nullptr;
+#endif
+    sodecl_lane_orbit(i, gid % SODECL_NL, buffer, t_state, y_state, params, counters, traj, newton, orbits, s0, nseg, final_snap, ckpt_t,
                       ckpt_y, ckpt_every, gstep0);
 }
 #endif

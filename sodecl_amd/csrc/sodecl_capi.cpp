@@ -123,7 +123,8 @@ ProgramKey make_key(const sodecl_ctx* ctx, int schedule, int group, int block, c
     // sizes of 128 and 512 lanes).
     FieldConfig field;
     const bool in_field = field_config(ctx, schedule, group, &field);
-    const int per_orbit = in_field ? field.lanes : schedule == 2 || schedule == 4 ? std::max(group, 1) : 1;
+    k.noise_lanes = noise_lanes(ctx, schedule, block);
+    const int per_orbit = in_field ? field.lanes : schedule == 2 || schedule == 4 ? std::max(group, 1) : k.noise_lanes;
     const long lanes = (long)ctx->orbits * per_orbit;
     k.field_lanes = field.lanes;
     k.field_cpl = field.cpl;
@@ -358,6 +359,20 @@ LaunchCfg choose_config(const sodecl_ctx* c)
 
 namespace sodecl_amd {
 
+// Small Euler-Maruyama launches of the lane schedule: as many lanes per orbit
+// (up to 16) as keep the launch at one wavefront per SIMD.  The reference's
+// launch design stays as it is, and so do systems whose noise would not fit
+// LDS comfortably.
+int noise_lanes(const sodecl_ctx* c, int schedule, int block)
+{
+    if (schedule != SODECL_SCHEDULE_LANE || c->solver != SODECL_STOCHASTIC_EULER ||
+        c->opts.schedule == SODECL_SCHEDULE_PLAIN || c->nnoi < 1 || c->nnoi > 16)
+        return 1;
+    int lanes = 1;
+    while (lanes < 16 && block % (2 * lanes) == 0 && (long)c->orbits * lanes * 2 <= 64L * 4 * device_cus(c)) lanes *= 2;
+    return lanes;
+}
+
 // The field form replaces the automatic pairwise choice (pairwise = 0) of the
 // default arithmetic: it sums the coupling through the components' features,
 // the strict arithmetic and the explicit pairwise layouts keep the pair terms.
@@ -438,7 +453,8 @@ int enqueue(sodecl_ctx* c, const LaunchCfg& cfg, double* t, double* y, const dou
         const int opb = cfg.block / cfg.group;
         grid = (unsigned)((orbits + opb - 1) / opb);
     } else {
-        grid = (unsigned)((orbits + cfg.block - 1) / cfg.block);
+        const int opb = cfg.block / noise_lanes(c, cfg.schedule, cfg.block);
+        grid = (unsigned)((orbits + opb - 1) / opb);
     }
     if (!ckpt_y || ckpt_every <= 0) {
         ckpt_y = nullptr;

@@ -60,6 +60,7 @@ struct ProgramKey {
     int newton_max_iter = 1000;
     double newton_tol = 0.0;     // > 0: _epsilon1_ in place of the reference's 1e-07
     int fp_contract = 0;
+    int noise_lanes = 1;         // lane schedule, Euler-Maruyama: lanes that draw an orbit's noise
     int field_lanes = 0;         // group schedule in field form: lanes per orbit (0: not in field form),
     int field_cpl = 0;           //   components per lane
     int field_block = 0;         //   and threads per block of its kernels
@@ -193,6 +194,8 @@ struct FieldConfig {
     int lanes = 0, cpl = 0, block = 0;
 };
 bool field_config(const sodecl_ctx* c, int schedule, int group, FieldConfig* f);
+// Lanes per orbit of the lane schedule (device/integrators.hip, SODECL_NL).
+int noise_lanes(const sodecl_ctx* c, int schedule, int block);
 // Program for the given schedule on the context's device (compiled on first use).
 std::shared_ptr<Program> get_program(sodecl_ctx* ctx, int schedule, int group, int block,
                                      const std::string& extra_defines = std::string());
