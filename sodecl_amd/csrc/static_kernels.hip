@@ -7,7 +7,9 @@
 #include <string>
 
 #include "../../include/sodecl.h"
+#include "device/sin.hip"
 #include "device/random.hip"
+#include "device/gauss.hip"
 #include "sodecl_internal.hpp"
 
 // ---------------------------------------------------------------------------
@@ -130,43 +132,83 @@ extern "C" int sodecl_threefry_device(const uint64_t* in, uint64_t* out, size_t 
 // from one Threefry-2x64-20 block with counter {row, col} and key
 // {seed, SODECL_SAMPLE_KEY1}, so every entry is reproducible on its own
 // whatever the launch shape.  u0, u1 = open-open (0, 1) doubles of the two
-// output words.  The distributions of up to 64 columns travel by value in
+// output words.  The distributions of up to 120 columns travel by value in
 // the kernel arguments (no device allocation; wider tables take several
 // launches).
+//
+// Bound by VALU issue: 110 instructions of Threefry per entry and 30 to 120 of
+// the distribution's functions against 8 bytes written.  With consecutive
+// entries of a row on consecutive lanes, a wavefront of a mixed table ran
+// every distribution's code for each of its entries (526 instructions per
+// entry, 262144 x 65 entries in 251 us).  Here a wavefront draws 64 rows of one
+// column, whose distribution is then the same for all its lanes, and a block
+// gathers its rows in LDS so that they leave as whole cache lines; the
+// logarithms of the log-uniform bounds are taken once per block, and the
+// normal columns use the noise's logarithm and cosine (gauss.hip).
 #define SODECL_SAMPLE_KEY1 0x5EEDD15C0FFEE5EDull
-#define SODECL_SAMPLE_CHUNK 64
+#define SODECL_SAMPLE_CHUNK 120   // its tile of 64 rows stays below 64 KiB
+#define SODECL_SAMPLE_WAVES 4
 
 struct sodecl_dist_chunk {
     sodecl_dist d[SODECL_SAMPLE_CHUNK];
     int c0, nc;   // first column, columns in this chunk
+    int groups;   // 64-row groups of a block's tile
 };
 
-__global__ void __launch_bounds__(256) sodecl_sample(const sodecl_dist_chunk chunk, int rows, int cols,
-                                                     unsigned long long seed, double* __restrict__ out)
+__global__ void __launch_bounds__(64 * SODECL_SAMPLE_WAVES)
+sodecl_sample(const sodecl_dist_chunk chunk, int rows, int cols, unsigned long long seed, double* __restrict__ out)
 {
-    const long long n = (long long)rows * chunk.nc;
-    const long long stride = (long long)gridDim.x * blockDim.x;
-    for (long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += stride) {
-        const int row = (int)(e / chunk.nc);
-        const int k = (int)(e - (long long)row * chunk.nc);
-        const int col = chunk.c0 + k;
-        const sodecl_dist d = chunk.d[k];
-        double v = d.a;
-        if (d.kind != SODECL_DIST_CONSTANT) {
-            sodecl_u64 w0, w1;
-            sodecl_threefry2x64_20((sodecl_u64)row, (sodecl_u64)col, (sodecl_u64)seed, SODECL_SAMPLE_KEY1, &w0, &w1);
-            const double u0 = sodecl_u01(w0);
-            if (d.kind == SODECL_DIST_UNIFORM) {
-                v = fma(d.b - d.a, u0, d.a);
-            } else if (d.kind == SODECL_DIST_LOG_UNIFORM) {
-                const double la = log(d.a);
-                v = exp(fma(log(d.b) - la, u0, la));
-            } else {   // normal: Box-Muller, cosine branch
-                const double u1 = sodecl_u01(w1);
-                v = fma(d.b, sqrt(-2.0 * log(u0)) * cos(2.0 * M_PI * u1), d.a);
+    extern __shared__ double sample_lds[];
+    const int nc = chunk.nc, pitch = nc | 1;   // odd: the lanes' rows fall on different banks
+    double* const bound = sample_lds;          // per column log a, log b - log a
+    double* const tile = sample_lds + 2 * nc;  // [64 * groups][pitch]
+    for (int k = threadIdx.x; k < nc; k += blockDim.x) {
+        const bool lu = chunk.d[k].kind == SODECL_DIST_LOG_UNIFORM;
+        const double la = lu ? log(chunk.d[k].a) : 0.0;
+        bound[2 * k] = la;
+        bound[2 * k + 1] = lu ? log(chunk.d[k].b) - la : 0.0;
+    }
+    __syncthreads();
+    const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    const int tile_rows = 64 * chunk.groups;
+    // this thread's entries of a tile in row order: its first, and the distance to the next
+    const int first_r = (int)threadIdx.x / nc, first_k = (int)threadIdx.x % nc;
+    const int step_r = (int)blockDim.x / nc, step_k = (int)blockDim.x % nc;
+    for (long long r0 = (long long)blockIdx.x * tile_rows; r0 < rows; r0 += (long long)gridDim.x * tile_rows) {
+        for (int u = wave; u < nc * chunk.groups; u += SODECL_SAMPLE_WAVES) {
+            const int k = u / chunk.groups, r = u % chunk.groups * 64 + lane;
+            const int kind = chunk.d[k].kind;
+            const double a = chunk.d[k].a, b = chunk.d[k].b;
+            double v = a;
+            if (kind != SODECL_DIST_CONSTANT) {
+                sodecl_u64 w0, w1;
+                sodecl_threefry2x64_20((sodecl_u64)(r0 + r), (sodecl_u64)(chunk.c0 + k), (sodecl_u64)seed,
+                                       SODECL_SAMPLE_KEY1, &w0, &w1);
+                const double u0 = sodecl_u01(w0);
+                if (kind == SODECL_DIST_UNIFORM) {
+                    v = fma(b - a, u0, a);
+                } else if (kind == SODECL_DIST_LOG_UNIFORM) {
+                    v = exp(fma(bound[2 * k + 1], u0, bound[2 * k]));
+                } else {   // normal: Box-Muller, cosine branch
+                    double s, c;
+                    sodecl_sincos_reduced(2.0 * M_PI * sodecl_u01(w1), &s, &c);
+                    v = fma(b, sqrt(-2.0 * sodecl_log_positive(u0)) * c, a);
+                }
+            }
+            tile[r * pitch + k] = v;
+        }
+        __syncthreads();
+        const int here = (int)min((long long)tile_rows, rows - r0);
+        for (int r = first_r, k = first_k; r < here;) {
+            out[(size_t)(r0 + r) * cols + chunk.c0 + k] = tile[r * pitch + k];
+            r += step_r;
+            k += step_k;
+            if (k >= nc) {
+                k -= nc;
+                ++r;
             }
         }
-        out[(size_t)row * cols + col] = v;
+        __syncthreads();   // before the next tile
     }
 }
 
@@ -189,12 +231,16 @@ extern "C" int sodecl_sample_device(const sodecl_dist* dists, int rows, int cols
         chunk.c0 = c0;
         chunk.nc = cols - c0 < SODECL_SAMPLE_CHUNK ? cols - c0 : SODECL_SAMPLE_CHUNK;
         for (int k = 0; k < chunk.nc; ++k) chunk.d[k] = dists[c0 + k];
-        const long long n = (long long)rows * chunk.nc;
-        long long blocks = (n + 255) / 256;
-        const long long cap = (long long)cus * 16;
+        // a narrow chunk takes several 64-row groups per tile, so that each of
+        // a block's wavefronts has a few columns' worth of draws between barriers
+        chunk.groups = chunk.nc >= 16 ? 1 : (16 + chunk.nc - 1) / chunk.nc;
+        const long long tile_rows = 64LL * chunk.groups;
+        long long blocks = (rows + tile_rows - 1) / tile_rows;
+        const long long cap = (long long)cus * 8;
         if (blocks > cap) blocks = cap;
-        hipLaunchKernelGGL(sodecl_sample, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, chunk, rows,
-                           cols, seed, out);
+        const size_t lds = (2 * (size_t)chunk.nc + (size_t)tile_rows * (chunk.nc | 1)) * sizeof(double);
+        hipLaunchKernelGGL(sodecl_sample, dim3((unsigned)blocks), dim3(64 * SODECL_SAMPLE_WAVES), lds,
+                           (hipStream_t)stream, chunk, rows, cols, seed, out);
         if (hipGetLastError() != hipSuccess) return 0;
     }
     return 1;
