@@ -167,7 +167,7 @@ SODECL_INLINE void sodecl_field_step(double t, double (&y)[SODECL_FC], sodecl_fi
     }
     sodecl_field_eval(t + _m_dt_, x, pp, lane, phi, sum, f);
 #pragma unroll
-    for (int c = 0; c < SODECL_FC; ++c) y[c] = y[c] + SODECL_RK4_DIV6((acc[c] + f[c]) * _m_dt_);
+    for (int c = 0; c < SODECL_FC; ++c) y[c] = y[c] + SODECL_RK4_UPDATE(acc[c] + f[c]);
 }
 #else
 // Euler-Maruyama (stochastic_euler.cl:10-22) with this lane's noise z.

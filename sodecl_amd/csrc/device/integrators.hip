@@ -66,13 +66,13 @@ SODECL_INLINE double sodecl_div(double a, double d, double rd)
 }
 
 // (a dt) / 6.00 of the RK4 update (rk4.cl:60): under strict arithmetic the
-// correctly rounded quotient, otherwise the product with the rounded
-// reciprocal (within an ulp of it; the same size of rounding change as
-// contraction, and right for infinities, NaN and signed zeros).
+// correctly rounded quotient of the rounded product, otherwise one product
+// with the constant dt / 6 (within two ulps of it; the same size of rounding
+// change as contraction, and right for infinities, NaN and signed zeros).
 #if SODECL_STRICT
-#define SODECL_RK4_DIV6(a) sodecl_div((a), 6.00, 1.0 / 6.00)
+#define SODECL_RK4_UPDATE(a) sodecl_div((a) * _m_dt_, 6.00, 1.0 / 6.00)
 #else
-#define SODECL_RK4_DIV6(a) ((a) * (1.0 / 6.00))
+#define SODECL_RK4_UPDATE(a) ((a) * (_m_dt_ / 6.00))
 #endif
 
 // The reference keeps the per-orbit counter as a double and assigns it to the
@@ -289,7 +289,7 @@ SODECL_INLINE int sodecl_lane_step(double t, double* y, double* yout, double* p)
     }
     SODECL_RHS(t + _m_dt_, x, k, p);
     SODECL_UNROLL
-    for (int i = 0; i < _numeq_; ++i) yout[i] = y[i] + SODECL_RK4_DIV6((yout[i] + k[i]) * _m_dt_);
+    for (int i = 0; i < _numeq_; ++i) yout[i] = y[i] + SODECL_RK4_UPDATE(yout[i] + k[i]);
     return 0;
 }
 #elif SODECL_IS_IMPLICIT
@@ -485,10 +485,12 @@ sodecl_lane(double* __restrict__ t_state, double* __restrict__ y_state, const do
 // state and stepping it with the same arithmetic as the lane schedule; the
 // plugin's sode_system_team shares the drift's costly terms among the team.
 // This multiplies the wavefronts of a launch by G at the cost of the work the
-// team duplicates, which pays only when the shared terms dominate the step
-// and the orbits leave SIMDs idle (for the oculomotor model, whose two burst
-// curves are about half of an RK4 step, it does not: 4.4e10 against 6.1e10
-// orbit-steps/s for 65536 orbits).  Lane l of a team stores components m with
+// team duplicates, which pays when the shared terms are a large part of the
+// step and the orbits leave SIMDs idle: the oculomotor model's two
+// exponentials per drift on two lanes are 230 instead of 283 VALU instructions
+// per RK4 step, 1.82 against 2.21 ms per 4000 steps up to 16384 orbits (the
+// automatic choice there), but 3.8 against 2.5 ms for 65536 orbits, which fill
+// every SIMD by themselves.  Lane l of a team stores components m with
 // m % G == l.  Arguments as sodecl_lane (explicit, non-stochastic solvers).
 // ---------------------------------------------------------------------------
 #if SODECL_SCHEDULE == 4 && (SODECL_SOLVER == 1 || SODECL_SOLVER == 2)
@@ -524,19 +526,28 @@ sodecl_team(double* __restrict__ t_state, double* __restrict__ y_state, const do
             for (int m = 0; m < _numeq_; ++m)
                 if (m % SODECL_GROUP == lane) o[(size_t)m * orbits] = y[m];
         }
-        for (int it = 0; it < _numsteps_; ++it, ++g) {
-            if (ckpt_y && g == ck_step) {
-                const long long k = ck++;
-                ck_step += ckpt_every;
-                SODECL_UNROLL
-                for (int m = 0; m < _numeq_; ++m)
-                    if (m % SODECL_GROUP == lane) ckpt_y[(size_t)k * slab + (size_t)m * orbits + i] = y[m];
-                if (lane == 0) ckpt_t[(size_t)k * orbits + i] = t;
+        // in runs that end at the next checkpoint, as in the lane schedule
+        for (int it = 0; it < _numsteps_;) {
+            int run = _numsteps_ - it;
+            if (ckpt_y) {
+                if (g == ck_step) {
+                    const long long k = ck++;
+                    ck_step += ckpt_every;
+                    SODECL_UNROLL
+                    for (int m = 0; m < _numeq_; ++m)
+                        if (m % SODECL_GROUP == lane) ckpt_y[(size_t)k * slab + (size_t)m * orbits + i] = y[m];
+                    if (lane == 0) ckpt_t[(size_t)k * orbits + i] = t;
+                }
+                if (ck_step - g < run) run = (int)(ck_step - g);   // g < ck_step here
             }
-            sodecl_lane_step(t, y, yn, p);
-            t = t + _m_dt_;
-            SODECL_UNROLL
-            for (int m = 0; m < _numeq_; ++m) y[m] = yn[m];
+            it += run;
+            g += run;
+            for (; run > 0; --run) {
+                sodecl_lane_step(t, y, yn, p);
+                t = t + _m_dt_;
+                SODECL_UNROLL
+                for (int m = 0; m < _numeq_; ++m) y[m] = yn[m];
+            }
         }
     }
     SODECL_UNROLL
@@ -819,7 +830,7 @@ SODECL_INLINE void sodecl_group_step(double t, double (&y)[SODECL_CPL], double (
     SODECL_EVAL(t + _m_dt_, xs[buf][slot], f);
 #pragma unroll
     for (int c = 0; c < SODECL_CPL; ++c)
-        if (lane + c * SODECL_G < _numeq_) y[c] = y[c] + SODECL_RK4_DIV6((acc[c] + f[c]) * _m_dt_);
+        if (lane + c * SODECL_G < _numeq_) y[c] = y[c] + SODECL_RK4_UPDATE(acc[c] + f[c]);
     buf ^= 1;
 }
 #endif

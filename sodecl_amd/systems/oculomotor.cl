@@ -98,8 +98,8 @@ double ocu_burst(double x, double a, double b, double at, double bt)
 }
 
 /* Both burst curves of the right-hand side, B(x) and B(-x), with their
- * shared work done once.  For x > 0, B(x) is on its saturating side with
- * exponent (-x)/bt = -|x|/bt and B(-x) on its ramp side with exponent
+ * shared work done once, from es = exp(-|x|/bt) and er = exp(-|x|/b).  For
+ * x > 0, B(x) is on its saturating side with exponent (-x)/bt = -|x|/bt and B(-x) on its ramp side with exponent
  * (-x)/b = -|x|/b; for x < 0 the two swap; for a zero x both are ramps whose
  * exponent is a zero, whose exp is 1 like exp(-|x|/b).  Every case therefore
  * needs exactly exp(-|x|/bt) and exp(-|x|/b).  The saturating value
@@ -107,14 +107,25 @@ double ocu_burst(double x, double a, double b, double at, double bt)
  * values -(a/b) x exp(-|x|/b) of B(x) and -(a/b) (-x) exp(-|x|/b) of B(-x)
  * are negatives of each other bit for bit (rounding to nearest is symmetric
  * in sign).  Each result has the bits of ocu_burst's. */
-void ocu_burst_pair(double x, double a, double b, double at, double bt, double* bx, double* bmx)
+void ocu_burst_pair(double x, double a, double b, double at, double bt, double es, double er, double* bx, double* bmx)
 {
-    double es, er;
-    ocu_exps(x, b, bt, &es, &er);
+#if defined(SODECL_STRICT) && !SODECL_STRICT
+    /* the GPU's default arithmetic: the curve that is not saturating is
+     * (a/b) |x| exp(-|x|/b) on either side, so one comparison places both
+     * (at x = 0 both values are zeros), and at (1 - e) is one fused
+     * multiply-add; a/b is written as the product with the reciprocal it
+     * becomes where 1/b is at hand, which not every kernel's compiler sees */
+    const int pos = x > 0;
+    const double sat = fma(-at, es, at);
+    const double ramp = (a * (1.0 / b)) * fabs(x) * er;
+    *bx = pos ? sat : ramp;
+    *bmx = pos ? ramp : sat;
+#else
     const double sat = at * (1.00 - es);
     const double ramp = -(a / b) * x * er;
     *bx = x > 0 ? sat : ramp;
     *bmx = x < 0 ? sat : -ramp;
+#endif
 }
 
 /* d(ocu_burst)/dx */
@@ -140,32 +151,51 @@ void ocu_rhs(double y[_numeq_], double yout[_numeq_], double p[_numpar_], double
     const double drive = y[3] - y[4];
 
     yout[0] = y[1];
+#if defined(SODECL_STRICT) && !SODECL_STRICT
+    /* the GPU's default arithmetic: the inhibition's common factor once, and
+     * every product that feeds a sum as the fused multiply-add it becomes
+     * anyway (left to the compiler, the choice among a sum's products may
+     * differ between the kernels, and their bits with it) */
+    const double cross = p[3] * y[3] * y[4];
+    yout[1] = fma(rate_sum, drive, fma(rate_prod, y[2], fma(-rate_prod, y[0], -(rate_sum * y[1]))));
+    yout[2] = fma(-y[2], 1.0 / OCU_TN, drive);
+    yout[3] = (1.00 / p[2]) * (fma(-cross, y[4], -y[3]) + br);
+    yout[4] = (1.00 / p[2]) * (fma(-cross, y[3], -y[4]) + bl);
+#else
     yout[1] = -(rate_sum * y[1]) - (rate_prod * y[0]) + (rate_prod * y[2]) + rate_sum * drive;
     yout[2] = -ocu_div(y[2], OCU_TN, 1.0 / OCU_TN) + drive;
     yout[3] = (1.00 / p[2]) * (-y[3] - (p[3] * y[3] * y[4] * y[4]) + br);
     yout[4] = (1.00 / p[2]) * (-y[4] - (p[3] * y[4] * y[3] * y[3]) + bl);
+#endif
     yout[5] = -drive;
 }
 
 void sode_system(double t, double y[_numeq_], double yout[_numeq_], double p[_numpar_])
 {
-    double br, bl;
-    ocu_burst_pair(y[5], p[0], p[1], p[4], p[5], &br, &bl);
+    double br, bl, es, er;
+    ocu_exps(y[5], p[1], p[5], &es, &er);
+    ocu_burst_pair(y[5], p[0], p[1], p[4], p[5], es, er, &br, &bl);
     ocu_rhs(y, yout, p, br, bl);
 }
 
 #ifdef SODECL_TEAM_API
-/* Team form of sode_system for the team schedule: the two burst curves, each
- * an exponential and most of the cost of the right-hand side, go to the two
- * lanes of a pair (even lane B(y5), odd lane B(-y5)) and are swapped between
- * them; every lane then forms the whole right-hand side.  The operations are
- * those of sode_system. */
+/* Team form of sode_system for the team schedule: the two exponentials, most
+ * of the right-hand side, go to the two lanes of a pair (even lane exp(-|x|/bt),
+ * odd lane exp(-|x|/b), one instruction stream with each lane's own
+ * reciprocal) and are swapped between them; every lane then forms the whole
+ * right-hand side.  The operations are those of sode_system. */
 void sode_system_team(double t, double y[_numeq_], double yout[_numeq_], double p[_numpar_])
 {
     const int odd = sodecl_lane() & 1;
-    const double mine = ocu_burst(odd ? -y[5] : y[5], p[0], p[1], p[4], p[5]);
+    /* (2/bt)*0.5 is exactly 1/bt: written so, the two candidates are not one
+     * division of a selected denominator */
+    const double rb = 1.0 / p[1];
+    const double rbt = (2.0 / p[5]) * 0.5;
+    const double mine = exp(ocu_div(-fabs(y[5]), odd ? p[1] : p[5], odd ? rb : rbt));
     const double other = sodecl_group_xor(mine, 1);
-    ocu_rhs(y, yout, p, odd ? other : mine, odd ? mine : other);
+    double br, bl;
+    ocu_burst_pair(y[5], p[0], p[1], p[4], p[5], odd ? other : mine, odd ? mine : other, &br, &bl);
+    ocu_rhs(y, yout, p, br, bl);
 }
 #endif
 
