@@ -23,6 +23,41 @@
 #define SODECL_NO_CONTRACT
 #endif
 
+// n / d correctly rounded for d in [1.7, 2.5] and |n| < 1/2, a multiple of
+// 2^-54; and the correctly rounded square root of a double in [2^-53, 128].
+// On the GPU they are the IEEE division's and square root's own refinement
+// steps, from the hardware's estimates on, without the scaling and the special
+// cases that these arguments do not need (the same bits, three and six
+// instructions fewer; tests compare both with the host's).
+SODECL_MATH_FN double sodecl_quotient_near(double n, double d)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    double r = __builtin_amdgcn_rcp(d);
+    r = fma(r, fma(-d, r, 1.0), r);
+    r = fma(r, fma(-d, r, 1.0), r);
+    const double q = n * r;
+    return fma(fma(-d, q, n), r, q);
+#else
+    return n / d;
+#endif
+}
+SODECL_MATH_FN double sodecl_sqrt_near(double x)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    SODECL_NO_CONTRACT
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y;
+    double h = 0.5 * y;
+    const double e = fma(-h, g, 0.5);
+    h = fma(h, e, h);
+    g = fma(g, e, g);
+    g = fma(fma(-g, g, x), h, g);
+    return fma(fma(-g, g, x), h, g);
+#else
+    return sqrt(x);
+#endif
+}
+
 // log u for a positive normal double u.
 // Method: u = 2^k m with m in [sqrt(1/2), sqrt(2)), f = m - 1 (exact), and
 // log m = 2 atanh s with s = f / (2 + f), |s| <= 3 - 2 sqrt 2 (Cody and
@@ -43,7 +78,7 @@ SODECL_MATH_FN double sodecl_log_positive(double u)
     const double m = ldexp(m0, low);
     const double dk = (double)(e - low);                  // u = 2^k m
     const double f = m - 1.0;
-    const double s = f / (2.0 + f);
+    const double s = sodecl_quotient_near(f, 2.0 + f);
     const double z = s * s;
     double g = 0x1.0c0aff044a970p-3;
     g = sodecl_fma_k(g, z, 0x1.0fbde0f4ad17bp-3);
@@ -83,7 +118,7 @@ SODECL_MATH_FN double sodecl_log_positive(double u)
 SODECL_MATH_FN void sodecl_sincos_reduced(double x, double* sx, double* cx)
 {
     SODECL_NO_CONTRACT
-    const double kk = fma(x, 0x1.45f306dc9c883p-1, 0x1.8p52);
+    const double kk = sodecl_fma_k(x, 0x1.45f306dc9c883p-1, 0x1.8p52);
     const double q = kk - 0x1.8p52;
     const double r1 = fma(-q, 0x1.921fb54442d18p+0, x);
     const double r = fma(-q, 0x1.1a62633145c07p-54, r1);

@@ -99,7 +99,7 @@ SODECL_INLINE void sodecl_noise_pair(int orbit, sodecl_u64 word, double dtsqrt, 
     sodecl_threefry2x64_20((sodecl_u64)orbit, word, SODECL_RNG_KEY0, SODECL_RNG_KEY1, &w0, &w1);
     const double u0 = sodecl_u01(w0);
     const double u1 = sodecl_u01(w1);
-    const double r = sqrt(-2 * sodecl_log_positive(u0));
+    const double r = sodecl_sqrt_near(-2 * sodecl_log_positive(u0));
     double s, c;
     sodecl_sincos_reduced(2 * M_PI * u1, &s, &c);
     *z0 = (r * c) * dtsqrt;

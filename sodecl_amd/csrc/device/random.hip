@@ -66,9 +66,13 @@ SODECL_INLINE void sodecl_threefry2x64_20(sodecl_u64 c0, sodecl_u64 c1, sodecl_u
 }
 
 // 64-bit word -> double in the open interval (0, 1): (1 + (w >> 11)) * (2^53-1) * 2^-106,
-// the open-open 64->53 conversion of Random123's u01.h:129-131.
+// the open-open 64->53 conversion of Random123's u01.h:129-131.  The 53-bit
+// integer k = w >> 11 is put together from its 32-bit halves exactly, and
+// (k + 1) c, of which 1 + k is exact too, is one fused multiply-add k c + c.
 SODECL_INLINE double sodecl_u01(sodecl_u64 w)
 {
-    return (double)(1ull + (w >> 11)) * 0x1.fffffffffffffp-54;
+    const double c = 0x1.fffffffffffffp-54;
+    const sodecl_u64 k = w >> 11;
+    return fma(fma((double)(unsigned)(k >> 32), 0x1p32, (double)(unsigned)k), c, c);
 }
 

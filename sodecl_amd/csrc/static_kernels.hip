@@ -192,7 +192,7 @@ sodecl_sample(const sodecl_dist_chunk chunk, int rows, int cols, unsigned long l
                 } else {   // normal: Box-Muller, cosine branch
                     double s, c;
                     sodecl_sincos_reduced(2.0 * M_PI * sodecl_u01(w1), &s, &c);
-                    v = fma(b, sqrt(-2.0 * sodecl_log_positive(u0)) * c, a);
+                    v = fma(b, sodecl_sqrt_near(-2.0 * sodecl_log_positive(u0)) * c, a);
                 }
             }
             tile[r * pitch + k] = v;
