@@ -237,6 +237,82 @@ SODECL_INLINE void sodecl_tri_solve(Lo lo, Di di, Up up, V v, double (&x)[SODECL
     x[R - 1] = X;
 }
 
+#if SODECL_WINDOW
+// Two-level matrices: every row that is coupled to another is coupled only to
+// rows without couplings (known from the constant zeros; row 0 stands for the
+// next partition's and row R - 1 for the previous one's).  A chain of cells
+// with two species each has this form under the reference's index mapping.
+// Nothing needs eliminating then: every pivot is its diagonal element, the
+// uncoupled rows divide, and the others substitute.
+template <class Lo, class Up> SODECL_INLINE bool sodecl_two_level(Lo lo, Up up)
+{
+    const int R = SODECL_BR;
+    const auto leaf = [&](int j) { return sodecl_zero(up(j)) && sodecl_zero(lo(j)); };
+    bool two = true;
+#pragma unroll
+    for (int j = 0; j < R; ++j)
+        two = two && ((sodecl_zero(up(j)) || leaf((j + R - 1) % R)) && (sodecl_zero(lo(j)) || leaf((j + 1) % R)));
+    return two;
+}
+SODECL_INLINE bool sodecl_normal(double v) { return __builtin_amdgcn_class(v, 0x108); }
+// Changes a and b to such that their reciprocals were b/q and a/q, where a b is
+// no normal number: each one's power of two goes to the other; a zero, an
+// infinity or no number gets no number, as from its own reciprocal.
+SODECL_INLINE void sodecl_pivots_scaled(double* pa, double* pb, double* q)
+{
+    const double a = *pa, b = *pb;
+    const bool na = __builtin_amdgcn_class(a, 0x267), nb = __builtin_amdgcn_class(b, 0x267);   // zero, infinite, NaN
+    const double fa = na ? 1.0 : __builtin_amdgcn_frexp_mant(a), fb = nb ? 1.0 : __builtin_amdgcn_frexp_mant(b);
+    *q = fa * fb;
+    *pb = na ? __builtin_nan("") : __builtin_amdgcn_ldexp(fb, -__builtin_amdgcn_frexp_exp(a));
+    *pa = nb ? __builtin_nan("") : __builtin_amdgcn_ldexp(fa, -__builtin_amdgcn_frexp_exp(b));
+}
+// Solves such a system.  The reciprocals come in pairs, 1/a = b/(ab) and
+// 1/b = a/(ab): ten issue slots in place of fourteen (a reciprocal's estimate
+// takes four).  An orbit whose residual norm is no number gets no numbers (the
+// reference's sweep carries it through every row).
+template <class Lo, class Up>
+SODECL_INLINE void sodecl_two_level_solve(Lo lo, double (&di)[SODECL_BR], Up up, double (&v)[SODECL_BR], double err,
+                                          double (&x)[SODECL_BR], int lane)
+{
+    const int R = SODECL_BR, P = R > 1 ? R / 2 : 1;
+    double q[P];   // 1/di[j] = di[j ^ 1] / q[j / 2]
+    bool plain = !(err != err);
+    if (R == 1) q[0] = di[0];
+#pragma unroll
+    for (int k = 0; k < R / 2; ++k) {
+        q[k] = di[2 * k] * di[2 * k + 1];
+        plain = plain & sodecl_normal(q[k]);
+    }
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(!plain) != 0, 0)) {
+#pragma unroll
+        for (int j = 0; j < R; ++j) v[j] = err != err ? err : v[j];
+#pragma unroll
+        for (int k = 0; k < R / 2; ++k)
+            if (!sodecl_normal(q[k])) sodecl_pivots_scaled(&di[2 * k], &di[2 * k + 1], &q[k]);
+    }
+#pragma unroll
+    for (int k = 0; k < P; ++k) q[k] = sodecl_rcp(q[k]);
+    const auto inv = [&](int j) { return R > 1 ? di[(j ^ 1) % R] * q[j / 2] : q[0]; };
+    const auto leaf = [&](int j) { return sodecl_zero(up(j)) && sodecl_zero(lo(j)); };
+#pragma unroll
+    for (int j = 0; j < R; ++j)
+        if (leaf(j)) x[j] = v[j] * inv(j);
+    double before = 0.0, after = 0.0;   // the neighbouring partitions' last and first unknown
+    if (!sodecl_zero(up(0))) before = sodecl_pcr_neighbour(x[R - 1], lane, 1, true);
+    if (!sodecl_zero(lo(R - 1))) after = sodecl_pcr_neighbour(x[0], lane, 1, false);
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+        if (!leaf(j)) {
+            double s = v[j];
+            if (!sodecl_zero(up(j))) s = s - up(j) * (j > 0 ? x[j - 1 < 0 ? 0 : j - 1] : before);
+            if (!sodecl_zero(lo(j))) s = s - lo(j) * (j + 1 < R ? x[j + 1 < R ? j + 1 : 0] : after);
+            x[j] = s * inv(j);
+        }
+    }
+}
+#endif
+
 // The most steps of any orbit of the wavefront, in a scalar register.
 SODECL_INLINE int sodecl_wave_steps(int steps)
 {
@@ -366,14 +442,19 @@ __device__ SODECL_BATCH_ITEM_ATTR void sodecl_batch_item(const int* __restrict__
             const bool done = !live || sqrt(err) < _epsilon1_;
 #endif
             if (__all(done)) break;
-            // A residual that is not a number leaves no component a number
-            // (the reference's sweep carries it through every row).
-            if (__builtin_expect(__builtin_amdgcn_ballot_w64(err != err) != 0, 0)) {
+            const auto low = [&](int j) { return lo[j]; };
+            const auto upp = [&](int j) { return up[j]; };
+            if (sodecl_two_level(low, upp)) {
+                sodecl_two_level_solve(low, di, upp, r, err, x, lane);
+            } else {
+                // A residual that is not a number leaves no component a number
+                // (the reference's sweep carries it through every row).
+                if (__builtin_expect(__builtin_amdgcn_ballot_w64(err != err) != 0, 0)) {
 #pragma unroll
-                for (int c = 0; c < SODECL_BR; ++c) r[c] = err != err ? err : r[c];
+                    for (int c = 0; c < SODECL_BR; ++c) r[c] = err != err ? err : r[c];
+                }
+                sodecl_tri_solve(low, [&](int j) { return di[j]; }, upp, [&](int j) { return r[j]; }, x, lane);
             }
-            sodecl_tri_solve([&](int j) { return lo[j]; }, [&](int j) { return di[j]; }, [&](int j) { return up[j]; },
-                             [&](int j) { return r[j]; }, x, lane);
             if (!done) {
 #pragma unroll
                 for (int c = 0; c < SODECL_BR; ++c) gg[c] = gg[c] - x[c];

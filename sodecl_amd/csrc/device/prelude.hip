@@ -22,14 +22,16 @@ __device__ inline double sodecl_dpp(double v)
 #define SODECL_DPP_ROW_SHR(n) (0x110 + (n))   // lane i <- lane i - n within its 16-lane row (0 past the start)
 #define SODECL_DPP_ROW_SHL(n) (0x100 + (n))   // lane i <- lane i + n within its 16-lane row (0 past the end)
 
-// 1/b from the hardware reciprocal and two Newton-Raphson steps (within an
-// ulp, for solves that are not the reference's operation by operation).
+// 1/b from the hardware reciprocal r (relative error e = 1 - b r, below 2^-20)
+// and one step of third order, r + r (e + e^2), which leaves e^3 and the last
+// rounding (within an ulp, for solves that are not the reference's operation by
+// operation; one instruction less than two Newton-Raphson steps, and issue
+// bounds those solves).
 __device__ inline double sodecl_rcp(double b)
 {
-    double r = __builtin_amdgcn_rcp(b);
-    r = fma(r, fma(-b, r, 1.0), r);
-    r = fma(r, fma(-b, r, 1.0), r);
-    return r;
+    const double r = __builtin_amdgcn_rcp(b);
+    const double e = fma(-b, r, 1.0);
+    return fma(r, fma(e, e, e), r);
 }
 
 // A value known to be a zero when the kernel is compiled: a coefficient the
