@@ -711,15 +711,21 @@ int run_fast(sodecl_ctx* c, long launches, const LaunchCfg& cfg)
     long per = c->opts.segments_per_launch > 0 ? c->opts.segments_per_launch : launches;
     size_t budget_rows = std::max<size_t>(2, traj_budget(c) / (slab * sizeof(double)));
     if ((size_t)per + 1 > budget_rows) per = (long)(budget_rows / pipe) - 1;
-    // A trajectory of more than 64 MiB for host memory streams in chunks of
-    // about 16 MiB: chunk k integrates while earlier chunks cross PCIe into
-    // pinned memory and are copied into the caller's array by the host
-    // threads (one copy from device into pageable memory measured about
-    // 8.5 GB/s).  Three buffers let each stage run a chunk ahead of the
-    // next one's jitter.  A host share needs the single launch.
+    // A trajectory of more than 6 MiB for host memory streams in four chunks,
+    // or more of about 16 MiB: chunk k integrates while earlier chunks cross
+    // PCIe into pinned memory and are copied into the caller's array by the
+    // host threads (one copy from device into pageable memory measured about
+    // 8.5 to 20 GB/s).  Three buffers let each stage run a chunk ahead of the
+    // next one's jitter.  A host share needs the single launch.  Session,
+    // run and result of 16384 plain oculomotor orbits x 2000 RK4 steps, one
+    // launch and four, ms: 8.7 MB 3.53 3.24, 16.5 MB 3.83 3.20, 32 MB 4.65
+    // 3.29 (2000 orbits, 9.7 MB: 3.27 2.9 to 3.1; 300 orbits, 7.2 MB: 3.15
+    // 3.00; 4.7 MB: no difference); at 158 MB chunks of 8 MiB take 5.3 and of
+    // 16 MiB 4.5.
     const size_t snap_bytes = slab * sizeof(double);
-    if (host_orbits(c) == 0 && snap_bytes * (size_t)(launches + 1) > ((size_t)64 << 20))
-        per = std::min<long>(per, std::max<long>(1, (long)(((size_t)16 << 20) / snap_bytes)));
+    const size_t all_bytes = snap_bytes * (size_t)(launches + 1);
+    if (host_orbits(c) == 0 && all_bytes > ((size_t)6 << 20))
+        per = std::min<long>(per, std::max<long>(1, (long)(std::min((size_t)16 << 20, all_bytes / 4) / snap_bytes)));
     if (per < 1) per = 1;
     const bool single = per >= launches;
     const size_t rows = (size_t)std::min<long>(per, launches) + 1;
