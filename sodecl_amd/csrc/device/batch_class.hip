@@ -439,7 +439,10 @@ __device__ SODECL_BATCH_ITEM_ATTR void sodecl_batch_item(const int* __restrict__
 #if SODECL_SOLVER == 3
             const bool done = !live || err < _epsilon1_;
 #else
-            const bool done = !live || sqrt(err) < _epsilon1_;
+            // sqrt(err) < _epsilon1_ without the root, which the whole wavefront
+            // waited for (450 chains of 5 to 100 cells, Newton run to
+            // convergence: 468 -> 419 us)
+            const bool done = !live || err < SODECL_EPSILON1_SQUARED;
 #endif
             if (__all(done)) break;
             const auto low = [&](int j) { return lo[j]; };
@@ -582,7 +585,7 @@ __device__ SODECL_BATCH_ITEM_ATTR void sodecl_batch_item(const int* __restrict__
 #if SODECL_SOLVER == 3
             const bool done = !live || err < _epsilon1_;
 #else
-            const bool done = !live || sqrt(err) < _epsilon1_;
+            const bool done = !live || err < SODECL_EPSILON1_SQUARED;
 #endif
             if (__all(done)) break;
             sodecl_wave_sync();

@@ -126,13 +126,30 @@ long num_launches(double tspan, double dt, int ksteps)
     return n;
 }
 
+// The least double t with sqrt(t) >= eps > 0: rounding is monotonic, so for every
+// v (infinities and NaN included) sqrt(v) < eps just where v < t.
+double sqrt_threshold(double eps)
+{
+    double t = eps * eps;
+    while (std::sqrt(t) < eps) t = std::nextafter(t, HUGE_VAL);
+    while (t > 0 && std::sqrt(std::nextafter(t, 0.0)) >= eps) t = std::nextafter(t, 0.0);
+    return t;
+}
+
 // "#define _epsilon1_ 1e-07" as the reference prints it (sodeclmgr.cpp:424-430),
-// or the caller's Newton threshold written exactly.
+// or the caller's Newton threshold written exactly; and the threshold for the
+// implicit midpoint's squared norm.
 std::string epsilon_define(const ProgramKey& k)
 {
-    if (!(k.newton_tol > 0)) return "#define _epsilon1_ 1e-07\n";
-    char buf[64];
-    std::snprintf(buf, sizeof buf, "#define _epsilon1_ %.17g\n", k.newton_tol);
+    const double eps = k.newton_tol > 0 ? k.newton_tol : 1e-07;
+    const double t = sqrt_threshold(eps);
+    char buf[128];
+    int n = k.newton_tol > 0 ? std::snprintf(buf, sizeof buf, "#define _epsilon1_ %.17g\n", eps)
+                             : std::snprintf(buf, sizeof buf, "#define _epsilon1_ 1e-07\n");
+    if (std::isinf(t))
+        std::snprintf(buf + n, sizeof buf - n, "#define SODECL_EPSILON1_SQUARED __builtin_inf()\n");
+    else
+        std::snprintf(buf + n, sizeof buf - n, "#define SODECL_EPSILON1_SQUARED %a\n", t);
     return buf;
 }
 
