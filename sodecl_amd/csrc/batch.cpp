@@ -121,6 +121,11 @@ int lanes_for(int neq, int rows)
 
 // Lanes per orbit and form of every size class.
 //
+// A batch of at most one wavefront per SIMD asks for the whole register file
+// per wavefront: the classes' kernels run side by side, and the dispatcher then
+// cannot put two of their wavefronts on one SIMD while others idle
+// (450 orbits of 10, 74 and 200 equations: 419 -> 390 us).
+//
 // Windowed form (up to 512 equations): eight rows per lane when the whole
 // batch then has at least four wavefronts per SIMD, where instructions count
 // (32768 orbits of 32, 128 and 512 equations: 8.5 ms, against 9.1 ms with four
@@ -163,6 +168,12 @@ std::vector<BatchShape> batch_shapes(const sodecl_batch* b)
         }
         shapes.push_back(s);
     }
+    long items = 0;
+    for (size_t k = 0; k < shapes.size(); ++k) {
+        const long n = std::count(b->cls.begin(), b->cls.end(), (int)k);
+        items += (n + shapes[k].slots() - 1) / shapes[k].slots();
+    }
+    for (BatchShape& s : shapes) s.alone = !b->cls.empty() && items <= 4L * cus;
     return shapes;
 }
 

@@ -327,7 +327,10 @@ std::string assemble_batch_program(const std::string& system_source, const Progr
         o << "#define SODECL_BATCH_KERNEL sodecl_batch_" << c << "\n";
         o << "#define SODECL_BATCH_ITEM sodecl_cls" << c << "::sodecl_batch_item\n";
         o << "#define SODECL_BATCH_SLOTS " << classes[c].slots() << "\n";
-        o << "#define SODECL_BATCH_WAVES " << classes[c].waves << "\n";
+        if (classes[c].alone)
+            o << "#define SODECL_BATCH_WAVES 1, 1\n";
+        else
+            o << "#define SODECL_BATCH_WAVES " << classes[c].waves << "\n";
         o << kBatchKernelSource << "\n";
         o << "#undef SODECL_BATCH_KERNEL\n#undef SODECL_BATCH_ITEM\n#undef SODECL_BATCH_WAVES\n#undef SODECL_BATCH_SLOTS\n";
     }
