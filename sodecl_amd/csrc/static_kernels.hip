@@ -2,7 +2,9 @@
 // user's system is compiled at run time by hipRTC instead).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstddef>
+#include <cstring>
 #include <mutex>
 #include <string>
 
@@ -149,24 +151,26 @@ extern "C" int sodecl_threefry_device(const uint64_t* in, uint64_t* out, size_t 
 #define SODECL_SAMPLE_CHUNK 120   // its tile of 64 rows stays below 64 KiB
 #define SODECL_SAMPLE_WAVES 4
 
-struct sodecl_dist_chunk {
-    sodecl_dist d[SODECL_SAMPLE_CHUNK];
+template <int N> struct sodecl_dist_chunk {
+    sodecl_dist d[N];
     int c0, nc;   // first column, columns in this chunk
     int groups;   // 64-row groups of a block's tile
+    int per;      // columns of a block (blockIdx.y takes the next ones)
 };
 
-__global__ void __launch_bounds__(64 * SODECL_SAMPLE_WAVES)
-sodecl_sample(const sodecl_dist_chunk chunk, int rows, int cols, unsigned long long seed, double* __restrict__ out)
+template <int N> __global__ void __launch_bounds__(64 * SODECL_SAMPLE_WAVES)
+sodecl_sample(const sodecl_dist_chunk<N> chunk, int rows, int cols, unsigned long long seed, double* __restrict__ out)
 {
     extern __shared__ double sample_lds[];
-    const int nc = chunk.nc, pitch = nc | 1;   // odd: the lanes' rows fall on different banks
+    const int k0 = (int)blockIdx.y * chunk.per, c0 = chunk.c0 + k0;   // the block's first column
+    const int nc = min(chunk.per, chunk.nc - k0), pitch = nc | 1;     // odd: the lanes' rows fall on different banks
     double* const bound = sample_lds;          // per column log a, log b - log a
     double* const tile = sample_lds + 2 * nc;  // [64 * groups][pitch]
     for (int k = threadIdx.x; k < nc; k += blockDim.x) {
-        const bool lu = chunk.d[k].kind == SODECL_DIST_LOG_UNIFORM;
-        const double la = lu ? log(chunk.d[k].a) : 0.0;
+        const bool lu = chunk.d[k0 + k].kind == SODECL_DIST_LOG_UNIFORM;
+        const double la = lu ? log(chunk.d[k0 + k].a) : 0.0;
         bound[2 * k] = la;
-        bound[2 * k + 1] = lu ? log(chunk.d[k].b) - la : 0.0;
+        bound[2 * k + 1] = lu ? log(chunk.d[k0 + k].b) - la : 0.0;
     }
     __syncthreads();
     const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
@@ -177,12 +181,12 @@ sodecl_sample(const sodecl_dist_chunk chunk, int rows, int cols, unsigned long l
     for (long long r0 = (long long)blockIdx.x * tile_rows; r0 < rows; r0 += (long long)gridDim.x * tile_rows) {
         for (int u = wave; u < nc * chunk.groups; u += SODECL_SAMPLE_WAVES) {
             const int k = u / chunk.groups, r = u % chunk.groups * 64 + lane;
-            const int kind = chunk.d[k].kind;
-            const double a = chunk.d[k].a, b = chunk.d[k].b;
+            const int kind = chunk.d[k0 + k].kind;
+            const double a = chunk.d[k0 + k].a, b = chunk.d[k0 + k].b;
             double v = a;
             if (kind != SODECL_DIST_CONSTANT) {
                 sodecl_u64 w0, w1;
-                sodecl_threefry2x64_20((sodecl_u64)(r0 + r), (sodecl_u64)(chunk.c0 + k), (sodecl_u64)seed,
+                sodecl_threefry2x64_20((sodecl_u64)(r0 + r), (sodecl_u64)(c0 + k), (sodecl_u64)seed,
                                        SODECL_SAMPLE_KEY1, &w0, &w1);
                 const double u0 = sodecl_u01(w0);
                 if (kind == SODECL_DIST_UNIFORM) {
@@ -200,7 +204,7 @@ sodecl_sample(const sodecl_dist_chunk chunk, int rows, int cols, unsigned long l
         __syncthreads();
         const int here = (int)min((long long)tile_rows, rows - r0);
         for (int r = first_r, k = first_k; r < here;) {
-            out[(size_t)(r0 + r) * cols + chunk.c0 + k] = tile[r * pitch + k];
+            out[(size_t)(r0 + r) * cols + c0 + k] = tile[r * pitch + k];
             r += step_r;
             k += step_k;
             if (k >= nc) {
@@ -210,6 +214,39 @@ sodecl_sample(const sodecl_dist_chunk chunk, int rows, int cols, unsigned long l
         }
         __syncthreads();   // before the next tile
     }
+}
+
+// Launches columns [c0, c0 + nc) of the table, nc <= N.
+template <int N>
+static bool sample_chunk(const sodecl_dist* dists, int c0, int nc, int rows, int cols, unsigned long long seed,
+                         double* out, int cus, hipStream_t stream)
+{
+    sodecl_dist_chunk<N> chunk;
+    std::memset(&chunk, 0, sizeof chunk);
+    chunk.c0 = c0;
+    chunk.nc = nc;
+    std::memcpy(chunk.d, dists + c0, (size_t)nc * sizeof(sodecl_dist));
+    // a narrow chunk takes several 64-row groups per tile, so that each of
+    // a block's wavefronts has a few columns' worth of draws between barriers;
+    // a table of fewer row groups than SIMDs spreads its columns over blocks
+    // instead (down to one column per wavefront), since its time is one
+    // wavefront's chain of draws (one call and its completion, 65 columns:
+    // 300 rows 32.7 -> 30.4, 17000 rows 46.6 -> 40.4, 30000 rows 47.8 -> 45.1 us)
+    const long long row_groups = (rows + 63LL) / 64;
+    const bool small = row_groups < 4 * cus;
+    chunk.groups = small || nc >= 16 ? 1 : (16 + nc - 1) / nc;
+    chunk.per = nc;
+    if (small) {
+        const long long parts = (4LL * cus + row_groups - 1) / row_groups;
+        chunk.per = std::max(std::min(nc, SODECL_SAMPLE_WAVES), (int)((nc + parts - 1) / parts));
+    }
+    const long long tile_rows = 64LL * chunk.groups;
+    const long long blocks = std::min((rows + tile_rows - 1) / tile_rows, (long long)cus * 8);
+    const unsigned parts = (unsigned)((nc + chunk.per - 1) / chunk.per);
+    const size_t lds = (2 * (size_t)chunk.per + (size_t)tile_rows * (chunk.per | 1)) * sizeof(double);
+    hipLaunchKernelGGL(sodecl_sample<N>, dim3((unsigned)blocks, parts), dim3(64 * SODECL_SAMPLE_WAVES), lds, stream,
+                       chunk, rows, cols, seed, out);
+    return hipGetLastError() == hipSuccess;
 }
 
 extern "C" int sodecl_sample_device(const sodecl_dist* dists, int rows, int cols, unsigned long long seed,
@@ -226,22 +263,15 @@ extern "C" int sodecl_sample_device(const sodecl_dist* dists, int rows, int cols
     (void)hipGetDevice(&device);
     int cus = 256;
     (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device);
+    // (the distributions travel in the kernel's arguments, which the host copies
+    // at each launch: three sizes, 0.3 us less for 16 columns than for 120)
     for (int c0 = 0; c0 < cols; c0 += SODECL_SAMPLE_CHUNK) {
-        sodecl_dist_chunk chunk{};
-        chunk.c0 = c0;
-        chunk.nc = cols - c0 < SODECL_SAMPLE_CHUNK ? cols - c0 : SODECL_SAMPLE_CHUNK;
-        for (int k = 0; k < chunk.nc; ++k) chunk.d[k] = dists[c0 + k];
-        // a narrow chunk takes several 64-row groups per tile, so that each of
-        // a block's wavefronts has a few columns' worth of draws between barriers
-        chunk.groups = chunk.nc >= 16 ? 1 : (16 + chunk.nc - 1) / chunk.nc;
-        const long long tile_rows = 64LL * chunk.groups;
-        long long blocks = (rows + tile_rows - 1) / tile_rows;
-        const long long cap = (long long)cus * 8;
-        if (blocks > cap) blocks = cap;
-        const size_t lds = (2 * (size_t)chunk.nc + (size_t)tile_rows * (chunk.nc | 1)) * sizeof(double);
-        hipLaunchKernelGGL(sodecl_sample, dim3((unsigned)blocks), dim3(64 * SODECL_SAMPLE_WAVES), lds,
-                           (hipStream_t)stream, chunk, rows, cols, seed, out);
-        if (hipGetLastError() != hipSuccess) return 0;
+        const int nc = std::min(cols - c0, SODECL_SAMPLE_CHUNK);
+        const hipStream_t s = (hipStream_t)stream;
+        const bool ok = nc <= 16   ? sample_chunk<16>(dists, c0, nc, rows, cols, seed, out, cus, s)
+                        : nc <= 64 ? sample_chunk<64>(dists, c0, nc, rows, cols, seed, out, cus, s)
+                                   : sample_chunk<SODECL_SAMPLE_CHUNK>(dists, c0, nc, rows, cols, seed, out, cus, s);
+        if (!ok) return 0;
     }
     return 1;
 }

@@ -26,3 +26,13 @@ def test_sampler_tile_edges(rows, cols):
         else:
             np.testing.assert_allclose(got[:, c], ref[:, c], rtol=0, atol=64e-16 * max(abs(d[1]), abs(d[2])))
     assert (whole[rows * cols:] == -7.0).all()
+
+
+@pytest.mark.parametrize("rows,cols", [(20000, 17), (40000, 61), (65473, 64), (65472, 65), (66000, 5)])
+def test_sampler_column_splits(rows, cols):
+    """Tables on either side of the size up to which columns spread over
+    blocks, with columns that do not come out even, and of each chunk's width:
+    the uniform columns bit for bit."""
+    dists = [("uniform", float(c), c + 2.0) if c % 3 else ("constant", float(c)) for c in range(cols)]
+    got = sample(dists, rows, 77).cpu().numpy()
+    np.testing.assert_array_equal(got, Oracle("oculomotor").sample(table(dists), rows, 77))
