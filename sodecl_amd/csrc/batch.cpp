@@ -121,20 +121,27 @@ int lanes_for(int neq, int rows)
 
 // Lanes per orbit and form of every size class.
 //
-// A batch of at most one wavefront per SIMD asks for the whole register file
-// per wavefront: the classes' kernels run side by side, and the dispatcher then
-// cannot put two of their wavefronts on one SIMD while others idle
-// (450 orbits of 10, 74 and 200 equations: 419 -> 390 us).
-//
-// Windowed form (up to 512 equations): eight rows per lane when the whole
-// batch then has at least four wavefronts per SIMD, where instructions count
-// (32768 orbits of 32, 128 and 512 equations: 8.5 ms, against 9.1 ms with four
-// and 9.5 ms with two rows where the class allows it); smaller batches, whose
-// time is the longest orbit's chain of Newton iterations, spread each orbit over
-// more lanes, two rows each (450 orbits of 10, 74 and 200 equations: 0.43
-// against 0.60 ms).  The two cross between 8000 and 16000 orbits of 22 to 512
-// equations (3.4 and 6.8 wavefronts per SIMD).  A power of two of rows keeps the
-// parity of a row's index known to the compiler.
+// Windowed form (up to 512 equations), by the wavefronts per SIMD of the whole
+// batch:
+//  * up to three with eight rows per lane, one wavefront at a time on a SIMD (each
+//    asks for the whole register file): the classes' kernels run side by side and
+//    the dispatcher would put two wavefronts on one SIMD while others idle, and a
+//    SIMD works off its wavefronts, longest orbits first, faster one after another
+//    than stacked.  The time is then the longest chains of Newton iterations, which
+//    fewer rows per lane shorten: two rows, or four, if they keep the batch at two
+//    wavefronts per SIMD, else eight.  450 orbits of 10, 74 and 200 equations to
+//    convergence, us: 390 with two and four rows, 580 with eight, and 443 with four
+//    if stacked.  Chains of 32, 128 and 512 equations, 50 to 200 steps, ms with two,
+//    four and eight rows, and two rows stacked: 2000 orbits 0.64 0.64 0.62 0.79,
+//    3000 orbits 0.82 0.67 0.76 0.90, 6000 orbits 1.47 1.18 1.10 1.26;
+//    of 22, 66 and 140 equations: 2000 orbits 0.57 0.57 0.76 0.68, 6000 orbits 1.26
+//    1.18 0.97 1.11, 8000 orbits 1.58 1.43 1.29 1.38;
+//  * from three to four, four rows, stacked (8000 chains of 32, 128 and 512
+//    equations with two, four and eight rows: 1.47 1.28 1.39, one at a time 1.88
+//    1.50 1.40);
+//  * from four on, eight rows, where instructions count (32768 orbits of 32, 128 and
+//    512 equations: 7.6 ms, against 8.1 ms with four and 8.8 ms with two).
+// A power of two of rows keeps the parity of a row's index known to the compiler.
 //
 // Through LDS: 16 lanes up to 32 equations, 32 up to 128, else 64; the
 // 128-equation class ran 2.5-3% faster on 32 lanes (four rows per lane, four
@@ -146,18 +153,17 @@ std::vector<BatchShape> batch_shapes(const sodecl_batch* b)
     int cus = 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, b->device) != hipSuccess || cus <= 0)
         cus = 256;
-    double waves = 0.0;
+    const int reach = b->features.window_reach;   // 0: no windowed form
+    std::vector<long> count(b->class_neq.size(), 0);
     for (int c : b->cls)
-        if (c >= 0 && c < (int)b->class_neq.size()) waves += lanes_for(b->class_neq[c], 8) / 64.0;
-    const bool large = b->cls.empty() || waves >= 4.0 * 4 * cus;
-    std::vector<BatchShape> shapes;
-    for (int neq : b->class_neq) {
+        if (c >= 0 && c < (int)count.size()) ++count[c];
+    auto window = [&](int neq) { return reach >= 1 && reach <= 8 && lanes_for(neq, 8) <= 64; };
+    auto shape = [&](int neq, int rows) {
         BatchShape s;
         s.neq = neq;
-        const int reach = b->features.window_reach;   // 0: no windowed form
-        s.window = reach >= 1 && reach <= 8 && lanes_for(neq, 8) <= 64;
+        s.window = window(neq);
         if (s.window) {
-            s.rows = large ? 8 : 2;
+            s.rows = rows;
             while (s.rows < reach || lanes_for(neq, s.rows) > 64) s.rows *= 2;
             s.lanes = lanes_for(neq, s.rows);
             s.waves = 4;
@@ -166,14 +172,26 @@ std::vector<BatchShape> batch_shapes(const sodecl_batch* b)
             s.rows = (neq + s.lanes - 1) / s.lanes;
             s.waves = s.rows <= 2 || (s.lanes == 32 && s.rows <= 4) ? 4 : (s.lanes == 64 && s.rows <= 8) ? 3 : 2;
         }
-        shapes.push_back(s);
+        return s;
+    };
+    bool windows = true;
+    auto per_simd = [&](int rows) {
+        double waves = 0.0;
+        for (size_t k = 0; k < count.size(); ++k) waves += (double)count[k] * shape(b->class_neq[k], rows).lanes / 64.0;
+        return waves / (4.0 * cus);
+    };
+    for (int neq : b->class_neq) windows = windows && window(neq);
+    int rows = 8;
+    bool alone = false;
+    if (!b->cls.empty() && per_simd(8) < 4.0) {
+        rows = per_simd(8) > 3.0 ? 4 : per_simd(2) <= 2.0 ? 2 : per_simd(4) <= 2.0 ? 4 : 8;
+        alone = per_simd(8) <= 3.0 && (windows || per_simd(rows) <= 1.0);
     }
-    long items = 0;
-    for (size_t k = 0; k < shapes.size(); ++k) {
-        const long n = std::count(b->cls.begin(), b->cls.end(), (int)k);
-        items += (n + shapes[k].slots() - 1) / shapes[k].slots();
+    std::vector<BatchShape> shapes;
+    for (int neq : b->class_neq) {
+        shapes.push_back(shape(neq, rows));
+        shapes.back().alone = alone;
     }
-    for (BatchShape& s : shapes) s.alone = !b->cls.empty() && items <= 4L * cus;
     return shapes;
 }
 

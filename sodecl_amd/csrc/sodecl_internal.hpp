@@ -46,7 +46,7 @@ struct BatchShape {
     bool window = false;   // components in registers, neighbours by lane shifts
     int rows = 1;          // consecutive rows (and components) per lane
     int waves = 2;         // wavefronts per SIMD its register budget is sized for
-    bool alone = false;    // the whole batch has at most one wavefront per SIMD (occupancy hint)
+    bool alone = false;    // one wavefront at a time on a SIMD (occupancy hint)
     int slots() const { return 64 / lanes; }   // orbits per wavefront
 };
 

@@ -47,3 +47,19 @@ def test_plugin_without_windowed_form():
     got, src = run(cfg, source.replace("SODE_REACH", "REACH").replace("band_window", "band_at"))
     assert "#define SODECL_WINDOW 1" not in src
     assert check_against_oracle(cfg, *got, range(60)) <= 1
+
+
+# (cells, orbits, rows per lane, one wavefront at a time): two rows, four and eight
+# rows one at a time, four rows stacked (256 compute units)
+@pytest.mark.parametrize("cells,orbits,rows,alone", [((16, 64, 256), 2300, (2, 2, 8), True),
+                                                     ((16, 64, 256), 3000, (4, 4, 8), True),
+                                                     ((16, 64, 256), 6000, (8, 8, 8), True),
+                                                     ((16, 64, 256), 8300, (4, 4, 8), False)])
+def test_rows_by_wavefronts_per_simd(cells, orbits, rows, alone):
+    cfg = configs.brusselator_batch(orbits=orbits, seed=orbits, solver=3, cells=cells, smin=5, smax=15, ksteps=5,
+                                    newton_max_iter=5)
+    got, src = run(cfg)
+    lines = src.splitlines()
+    assert tuple(int(l.split()[2]) for l in lines if l.startswith("#define SODECL_BR ")) == rows
+    assert all(l.endswith(" 1, 1") == alone for l in lines if l.startswith("#define SODECL_BATCH_WAVES "))
+    assert check_against_oracle(cfg, *got, range(0, orbits, orbits // 40)) <= 1
