@@ -69,8 +69,8 @@ def parse():
 TRAFFIC_PROFILES = {
     "oculomotor_rk4": "oculomotor_rk4_hbm_traffic.md",
     "oculomotor_rk4_plain_plugin": "sodecl_lane_oculomotor_rk4_plain.md",
-    "kuramoto_euler": "sodecl_group_kuramoto_euler_n10.md",
-    "kuramoto_em": "sodecl_group_kuramoto_em_n32.md",
+    "kuramoto_euler": "sodecl_field_kuramoto_euler_n10.md",
+    "kuramoto_em": "sodecl_field_kuramoto_em_n32.md",
 }
 
 

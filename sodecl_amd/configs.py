@@ -32,6 +32,13 @@ SYSTEMS = os.path.join(HERE, "systems")
 OCULOMOTOR_DEFAULTS = np.array([120.0, 1.5, 0.0045, 0.05, 600.0, 9.0])
 
 
+def kuramoto_rhs_flops(n):
+    """FP64 flops of one drift of n coupled phases, a transcendental counted as
+    20: the coupling's sums over sin and cos of the phases (two transcendentals
+    and two additions per component) and dtheta_i = w_i + K/N (c_i S - s_i C)."""
+    return n * (2 * 20 + 2 + 6)
+
+
 def kuramoto_euler(orbits=1024, n=10, seed=0):
     rng = np.random.default_rng(seed)
     K = rng.uniform(0, 5, orbits)
@@ -40,7 +47,7 @@ def kuramoto_euler(orbits=1024, n=10, seed=0):
     return dict(name="kuramoto_euler", system=os.path.join(SYSTEMS, "kuramoto.cl"), solver=1, neq=n,
                 npar=n + 1, nnoi=0, orbits=orbits, dt=0.01, tspan=10.0, ksteps=10,
                 y0=theta0, params=np.concatenate([K[:, None], w], 1), counters=None,
-                flops_per_orbit_step=2 * n * n + 3 * n + 2 * n + 1 + 20 * n * n)
+                flops_per_orbit_step=kuramoto_rhs_flops(n) + 2 * n + 1)
 
 
 def oculomotor_rk4(orbits=65536, seed=0, dt=1e-3, tspan=20.0, ksteps=100):
@@ -71,9 +78,9 @@ def kuramoto_em(orbits=262144, n=32, seed=0, tspan=10.0, ksteps=100):
     params = np.concatenate([K[:, None], w, np.repeat(sigma[:, None], n, 1)], 1)
     counters = np.full(orbits, float(seed) * 2.0 ** 32)
     calls = (n + 1) // 2
-    # RHS 2N^2+3N, noise calls*(4 mul + sqrt) + N, stoch N, update 2N, t 1;
-    # transcendentals: N^2 sin + calls*(log + sincos)
-    flops = (2 * n * n + 3 * n) + calls * 9 + n + 2 * n + 2 * n + 1 + 20 * (n * n + 3 * calls)
+    # RHS, noise calls*(4 mul + sqrt) + N, stoch N, update 2N, t 1;
+    # transcendentals: calls*(log + sincos)
+    flops = kuramoto_rhs_flops(n) + calls * 9 + n + 2 * n + 2 * n + 1 + 20 * 3 * calls
     return dict(name="kuramoto_em", system=os.path.join(SYSTEMS, "kuramoto.cl"), solver=0, neq=n,
                 npar=2 * n + 1, nnoi=n, orbits=orbits, dt=1e-3, tspan=tspan, ksteps=ksteps, y0=theta0,
                 params=params, counters=counters, flops_per_orbit_step=flops)
@@ -84,7 +91,7 @@ def kuramoto_rk4(orbits=16384, n=64, seed=0, dt=0.01, tspan=20.0, ksteps=10):
     K = rng.uniform(0, 5, orbits)
     w = rng.normal(1.0, 0.1, (orbits, n))
     theta0 = rng.uniform(0, 2 * np.pi, (orbits, n))
-    rhs = 2 * n * n + 3 * n + 20 * n * n
+    rhs = kuramoto_rhs_flops(n)
     return dict(name="kuramoto_rk4", system=os.path.join(SYSTEMS, "kuramoto.cl"), solver=2, neq=n,
                 npar=n + 1, nnoi=0, orbits=orbits, dt=dt, tspan=tspan, ksteps=ksteps, y0=theta0,
                 params=np.concatenate([K[:, None], w], 1), counters=None,

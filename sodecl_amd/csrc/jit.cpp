@@ -153,12 +153,11 @@ std::string epsilon_define(const ProgramKey& k)
     return buf;
 }
 
-// sin(), sincos() and exp() of the system source resolve to sodecl_sin
-// (device/sin.hip), sodecl_sincos (device/sincos.hip) and sodecl_exp
-// (device/exp.hip) unless the caller asked for the device library's; the solver templates after the system source keep the library's
-// functions.
-// Text around the user's system source: the own sine and exponential in
-// place of the library's, and in the default arithmetic (fp_contract = 0)
+// Text around the user's system source: sin(), sincos() and exp() resolve to
+// sodecl_sin (device/sin.hip), sodecl_sincos (device/sincos.hip) and sodecl_exp
+// (device/exp.hip) unless the caller asked for the device library's (the solver
+// templates after the system source keep the library's functions), and in the
+// default arithmetic (fp_contract = 0)
 // divisions as products with reciprocals (a division by a value fixed over
 // the integration then costs one multiply per evaluation, its reciprocal
 // hoisted out of the step loop; each quotient within about an ulp of the

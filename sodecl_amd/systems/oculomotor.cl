@@ -99,9 +99,10 @@ double ocu_burst(double x, double a, double b, double at, double bt)
 
 /* Both burst curves of the right-hand side, B(x) and B(-x), with their
  * shared work done once, from es = exp(-|x|/bt) and er = exp(-|x|/b).  For
- * x > 0, B(x) is on its saturating side with exponent (-x)/bt = -|x|/bt and B(-x) on its ramp side with exponent
- * (-x)/b = -|x|/b; for x < 0 the two swap; for a zero x both are ramps whose
- * exponent is a zero, whose exp is 1 like exp(-|x|/b).  Every case therefore
+ * x > 0, B(x) is on its saturating side with exponent (-x)/bt = -|x|/bt and
+ * B(-x) on its ramp side with exponent (-x)/b = -|x|/b; for x < 0 the two swap;
+ * for a zero x both are ramps whose exponent is a zero, whose exp is 1 like
+ * exp(-|x|/b).  Every case therefore
  * needs exactly exp(-|x|/bt) and exp(-|x|/b).  The saturating value
  * at(1 - exp(-|x|/bt)) serves whichever curve is on that side, and the ramp
  * values -(a/b) x exp(-|x|/b) of B(x) and -(a/b) (-x) exp(-|x|/b) of B(-x)
