@@ -415,7 +415,7 @@ bool field_config(const sodecl_ctx* c, int schedule, int group, FieldConfig* f)
     *f = FieldConfig{};
     const bool automatic_lane = schedule == SODECL_SCHEDULE_LANE && c->opts.schedule == SODECL_SCHEDULE_AUTO &&
                                 !c->tuned_schedule && !c->tuning && c->opts.group_size <= 0 &&
-                                c->opts.block_size <= 0 && !(c->opts.host_share > 0) && c->neq >= 2;
+                                c->opts.block_size <= 0 && c->neq >= 2;
     if ((schedule != SODECL_SCHEDULE_GROUP && !automatic_lane) || !c->features.field || c->opts.pairwise != 0 ||
         c->opts.fp_contract)
         return false;

@@ -44,3 +44,27 @@ def test_explicit_choices_keep_the_lane_schedule(opts):
     assert "#define SODECL_USE_FIELD 1" not in s.program_source()
     ref = Oracle("kuramoto").run("rk4", cfg["y0"], cfg["params"], cfg["dt"], cfg["tspan"], cfg["ksteps"])
     assert_traj_close(out, ref["out"], what=str(opts))
+
+
+@pytest.mark.parametrize("solver", [0, 2])
+def test_host_share_beside_the_field_form(solver):
+    """The GPU's orbits of an automatic run have the bits of a run without host
+    share; the host's, which the lane arithmetic integrates, match the oracle."""
+    orbits, n = 200, 5
+    if solver == 0:
+        cfg = configs.kuramoto_em(orbits=orbits, n=n, seed=3, tspan=0.1, ksteps=10)
+    else:
+        cfg = configs.kuramoto_rk4(orbits=orbits, n=n, seed=3, dt=0.01, tspan=0.5, ksteps=5)
+    out = []
+    for share in (0.0, 0.3):
+        s = configs.session_for(cfg, host_share=share)
+        s.setup(cfg["y0"], cfg["params"], None, cfg.get("counters"))
+        out.append(s.run().reshape(s.nsnap, n, orbits))
+        assert "#define SODECL_USE_FIELD 1" in s.program_source()
+    assert s.host_stats()[1] == 60
+    np.testing.assert_array_equal(out[0][:, :, :140], out[1][:, :, :140])
+    ref = Oracle("kuramoto").run({0: "em", 2: "rk4"}[solver], cfg["y0"], cfg["params"], cfg["dt"], cfg["tspan"],
+                                 cfg["ksteps"], counters=cfg.get("counters"), nnoi=cfg["nnoi"])
+    assert_traj_close(out[1], ref["out"], what="host share")
+    if solver == 0:
+        np.testing.assert_array_equal(s.counters(), ref["counters"])
