@@ -244,6 +244,26 @@ SODECL_INLINE int sodecl_implicit_step(double t, double* y, double* yout, double
 }
 #endif  // SODECL_IS_IMPLICIT
 
+// Steps per block of the explicit solvers' step loop.  With one wavefront per
+// SIMD a step leaves issue slots empty; in one block the next step's terms that
+// need only the state's early components (the oculomotor model's exponentials
+// need one component, which the other components' drifts do not) start under
+// the step before, and the loop's scalar instructions are shared.  Oculomotor,
+// us with one, two, four and eight steps: RK4, 65536 orbits x 2000 steps 1329
+// 1284 1294 1294 (segments of 20 steps 1285 1313 1254 1293), 40000 x 2000
+// 1184 1122 1119 1119; Euler, 60000 x 2000 366 353 339 338; 5000 Euler-Maruyama
+// orbits x 1000 steps 335 324 319 309.  Segments of seven steps, with a rest,
+// gain less than a branching source loses (1921 1926 1976 1925), and noise
+// drawn for two steps at a time leaves nothing to unroll (534 553 558 557).
+#if defined(SODECL_ONE_WAVE) && _numeq_ <= 8 && _numsteps_ >= 8 && \
+    (SODECL_SOLVER == 1 || SODECL_SOLVER == 2 || (SODECL_IS_SDE && defined(SODECL_NL) && SODECL_NL >= 4))
+#define SODECL_STEP_BLOCKS 1
+#define SODECL_STEP_LOOP _Pragma("unroll 4")
+#else
+#define SODECL_STEP_BLOCKS 0
+#define SODECL_STEP_LOOP
+#endif
+
 // ---------------------------------------------------------------------------
 // One step of the selected solver with the whole state per lane (lane and
 // team schedules).  Under the team schedule the drift comes from the
@@ -326,6 +346,21 @@ SODECL_INLINE int sodecl_lane_step(double t, double* y, double* yout, double* p)
 #define SODECL_NOISE_ROW ((SODECL_NL * SODECL_NNOI_ALLOC) | 1)
 #endif
 
+#if SODECL_IS_SDE
+// Euler-Maruyama (stochastic_euler.cl:10-22)
+SODECL_INLINE void sodecl_em_step(double& t, double* y, double* yn, double* p, double* noise)
+{
+    double st[_numeq_];
+    sode_system(t, y, yn, p);
+    sode_system_stoch(t, y, st, p, noise);
+    SODECL_UNROLL
+    for (int m = 0; m < _numeq_; ++m) yn[m] = y[m] + yn[m] * _m_dt_ + st[m];
+    t = t + _m_dt_;
+    SODECL_UNROLL
+    for (int m = 0; m < _numeq_; ++m) y[m] = yn[m];
+}
+#endif
+
 // Orbit i of a lane-schedule launch: one lane of sodecl_lane (lane sub of its
 // SODECL_NL, with the orbit's noise buffer), or one iteration of the host
 // share's orbit loop (SODECL_HOST_BUILD).
@@ -381,10 +416,9 @@ SODECL_INLINE void sodecl_lane_orbit(int i, int sub, double* buffer, double* __r
             }
             it += run;
             g += run;
-            for (; run > 0; --run) {
-#if SODECL_IS_SDE
-                // Noise for this step (stochastic_solver_caller.cl:44-66)
 #if SODECL_NL > 1
+            while (run > 0) {
+                // the noise of the next SODECL_NL steps
                 if (drawn == SODECL_NL) {
                     sodecl_wave_sync();   // the buffer's last step has been read
                     const double first = cnt + (double)(sub * SODECL_CALLS);
@@ -397,10 +431,21 @@ SODECL_INLINE void sodecl_lane_orbit(int i, int sub, double* buffer, double* __r
                     sodecl_wave_sync();
                     drawn = 0;
                 }
-                for (int in = 0; in < _numnoi_; ++in) noise[in] = buffer[drawn * _numnoi_ + in];
-                ++drawn;
-                cnt = cnt + (double)calls;
+                int steps = run < SODECL_NL - drawn ? run : SODECL_NL - drawn;
+                run -= steps;
+                SODECL_STEP_LOOP
+                for (; steps > 0; --steps) {
+                    for (int in = 0; in < _numnoi_; ++in) noise[in] = buffer[drawn * _numnoi_ + in];
+                    ++drawn;
+                    cnt = cnt + (double)calls;
+                    sodecl_em_step(t, y, yn, p, noise);
+                }
+            }
 #else
+            SODECL_STEP_LOOP
+            for (; run > 0; --run) {
+#if SODECL_IS_SDE
+                // Noise for this step (stochastic_solver_caller.cl:44-66)
                 int nc = 0;
                 for (int in = 0; in < calls; ++in) {
                     double z0, z1;
@@ -409,22 +454,15 @@ SODECL_INLINE void sodecl_lane_orbit(int i, int sub, double* buffer, double* __r
                     if (nc < _numnoi_) noise[nc++] = z0;
                     if (nc < _numnoi_) noise[nc++] = z1;
                 }
-#endif
-                // Euler-Maruyama (stochastic_euler.cl:10-22)
-                {
-                    double st[_numeq_];
-                    sode_system(t, y, yn, p);
-                    sode_system_stoch(t, y, st, p, noise);
-                    SODECL_UNROLL
-                    for (int m = 0; m < _numeq_; ++m) yn[m] = y[m] + yn[m] * _m_dt_ + st[m];
-                }
+                sodecl_em_step(t, y, yn, p, noise);
 #else
                 nu += sodecl_lane_step(t, y, yn, p);
-#endif
                 t = t + _m_dt_;
                 SODECL_UNROLL
                 for (int m = 0; m < _numeq_; ++m) y[m] = yn[m];
+#endif
             }
+#endif
         }
     }
     if (sub != 0) return;
@@ -544,12 +582,21 @@ sodecl_team(double* __restrict__ t_state, double* __restrict__ y_state, const do
             }
             it += run;
             g += run;
-            for (; run > 0; --run) {
+            const auto step = [&]() {
                 sodecl_lane_step(t, y, yn, p);
                 t = t + _m_dt_;
                 SODECL_UNROLL
                 for (int m = 0; m < _numeq_; ++m) y[m] = yn[m];
+            };
+#if SODECL_STEP_BLOCKS
+            // two steps in a block (written out, since the compiler leaves loops
+            // with lane exchanges rolled): 16384 orbits x 4000 steps 1.99 -> 1.94 ms
+            for (; run > 1; run -= 2) {
+                step();
+                step();
             }
+#endif
+            for (; run > 0; --run) step();
         }
     }
     SODECL_UNROLL

@@ -208,7 +208,8 @@ std::string assemble_program(const std::string& system_source, const ProgramKey&
     if (k.field_lanes > 0)
         o << "#define SODECL_USE_FIELD 1\n#define SODECL_FIELD_API 1\n#define SODECL_FL " << k.field_lanes
           << "\n#define SODECL_FC " << k.field_cpl << "\n#define SODECL_FBLOCK " << k.field_block << "\n";
-    if (k.one_wave_per_simd) o << "#define SODECL_KERNEL_ATTR __attribute__((amdgpu_waves_per_eu(1, 1)))\n";
+    if (k.one_wave_per_simd)
+        o << "#define SODECL_ONE_WAVE 1\n#define SODECL_KERNEL_ATTR __attribute__((amdgpu_waves_per_eu(1, 1)))\n";
     o << k.extra_defines;
     // OpenCL C spellings a system source may use
     for (const char* kw : {"__kernel", "__global", "__private"})
