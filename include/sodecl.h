@@ -56,7 +56,7 @@ enum sodecl_output { SODECL_OUTPUT_NONE = 0, SODECL_OUTPUT_ARRAY = 1, SODECL_OUT
  * work-item per orbit and one launch per ksteps segment). */
 enum sodecl_schedule {
     SODECL_SCHEDULE_AUTO = 0,  /* group when the plugin has per-component entry points
-                                  and the system is large enough, else team for RK4 with a
+                                  and the system is large enough, else team for Euler and RK4 with a
                                   plugin that has the entry point and few orbits, else lane; timed
                                   choice (team included) when autotune is on */
     SODECL_SCHEDULE_LANE = 1,  /* one orbit per lane, state in registers */

@@ -310,12 +310,12 @@ LaunchCfg choose_config(const sodecl_ctx* c)
         sched = (group_possible(c) && c->neq >= 8) ? 2 : 1;
         // A plugin's team entry point shares the costly terms of an orbit's
         // drift between two lanes: fewer instructions per step for twice the
-        // lanes, which pays while those still have a SIMD each.  Oculomotor
-        // RK4, 4000 steps: 1.82 against 2.21 ms up to 16384 orbits, 2.09 against
-        // 2.23 ms at 32768, 3.8 against 2.5 ms at 65536 (Euler's step, with one
-        // drift, is no shorter).
-        if (sched == 1 && team_possible(c) && c->solver == SODECL_RUNGE_KUTTA && c->opts.group_size <= 0 &&
-            2L * c->orbits <= 64L * 4 * device_cus(c))
+        // lanes, which pays while those still have a SIMD each.  Oculomotor,
+        // 4000 steps: RK4 1.83 against 2.18 ms up to 16384 orbits, 2.02 against
+        // 2.20 ms at 32768, 3.6 against 2.4 ms at 65536; Euler 0.52 against 0.57,
+        // 0.56 against 0.59 and 1.00 against 0.64 ms.
+        if (sched == 1 && team_possible(c) && (c->solver == SODECL_RUNGE_KUTTA || c->solver == SODECL_EULER) &&
+            c->opts.group_size <= 0 && 2L * c->orbits <= 64L * 4 * device_cus(c))
             sched = 4;
     }
     if (sched == SODECL_SCHEDULE_GROUP && !group_possible(c)) sched = 1;
