@@ -117,11 +117,17 @@ __device__ inline double sodecl_group_sum(double v)
 //   sodecl_group_size()     lanes per orbit
 //   sodecl_lane()           this lane's index within the team, 0..G-1
 //   sodecl_group_xor(v, m)  v of team lane sodecl_lane() ^ m (m < G)
-// These exist only in device code compiled for the team schedule
+// These exist only in device code compiled for the team schedule, and for
+// Euler-Maruyama launches of the lane schedule whose orbits have several lanes
 // (SODECL_TEAM_API is defined there).
 #if SODECL_SCHEDULE == 4
-__device__ inline int sodecl_group_size() { return SODECL_GROUP; }
-__device__ inline int sodecl_lane() { return (int)(threadIdx.x % SODECL_GROUP); }
+#define SODECL_TEAM_LANES SODECL_GROUP
+#elif SODECL_SCHEDULE == 1 && defined(SODECL_NOISE_TEAM)
+#define SODECL_TEAM_LANES SODECL_NL
+#endif
+#ifdef SODECL_TEAM_LANES
+__device__ inline int sodecl_group_size() { return SODECL_TEAM_LANES; }
+__device__ inline int sodecl_lane() { return (int)(threadIdx.x % SODECL_TEAM_LANES); }
 // Lane exchange within quads by DPP quad permutations for m = 1, 2, 3
 // (no LDS traffic), cross-lane permute otherwise.
 __device__ inline double sodecl_group_xor(double v, int m)
@@ -130,7 +136,7 @@ __device__ inline double sodecl_group_xor(double v, int m)
     case 1: return sodecl_dpp<SODECL_DPP_XOR1>(v);
     case 2: return sodecl_dpp<SODECL_DPP_XOR2>(v);
     case 3: return sodecl_dpp<SODECL_DPP_XOR3>(v);
-    default: return __shfl_xor(v, m, SODECL_GROUP);
+    default: return __shfl_xor(v, m, SODECL_TEAM_LANES);
     }
 }
 #define SODECL_TEAM_API 1

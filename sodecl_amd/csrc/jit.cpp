@@ -205,6 +205,7 @@ std::string assemble_program(const std::string& system_source, const ProgramKey&
     o << "#define SODECL_HAS_JACOBIAN_EXACT " << (f.jacobian_exact ? 1 : 0) << "\n";
     o << "#define SODECL_USE_PAIRS " << (k.schedule == 2 && f.pairs ? k.use_pairs : 0) << "\n";
     if (k.noise_lanes > 1) o << "#define SODECL_NL " << k.noise_lanes << "\n";
+    if (k.noise_lanes > 1 && f.team) o << "#define SODECL_NOISE_TEAM 1\n";
     if (k.field_lanes > 0)
         o << "#define SODECL_USE_FIELD 1\n#define SODECL_FIELD_API 1\n#define SODECL_FL " << k.field_lanes
           << "\n#define SODECL_FC " << k.field_cpl << "\n#define SODECL_FBLOCK " << k.field_block << "\n";
