@@ -34,3 +34,17 @@ def test_segment_remainders(solver, schedule, ksteps):
     assert_traj_close(out, ref["out"], what=f"solver {solver} {schedule} ksteps {ksteps}")
     if solver == 0:
         np.testing.assert_array_equal(s.counters(), ref["counters"])
+
+
+@pytest.mark.parametrize("ksteps", [3, 4, 7, 9])
+def test_field_segment_remainders(ksteps):
+    """The field form's Euler steps with one component per lane."""
+    orbits, n, dt = 67, 10, 2.0 ** -7
+    tspan = 5 * ksteps * dt
+    cfg = configs.kuramoto_rk4(orbits=orbits, n=n, seed=ksteps, dt=dt, tspan=tspan, ksteps=ksteps)
+    s = si.Session(cfg["system"], 1, orbits, n, n + 1, 0, dt, tspan, ksteps, 0, {})
+    s.setup(cfg["y0"], cfg["params"])
+    out = s.run().reshape(s.nsnap, n, orbits)
+    assert "#define SODECL_FL 16\n#define SODECL_FC 1\n" in s.program_source()
+    ref = Oracle("kuramoto").run("euler", cfg["y0"], cfg["params"], dt, tspan, ksteps)
+    assert_traj_close(out, ref["out"], what=f"field Euler ksteps {ksteps}")
