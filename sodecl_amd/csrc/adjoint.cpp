@@ -45,13 +45,6 @@ int check_adjoint(sodecl_ctx* c, int& sched, int& group, int& block)
     return 1;
 }
 
-const char* adjoint_kernel(const sodecl_ctx* c, int sched, int group)
-{
-    FieldConfig field;
-    if (implicit(c)) return "sodecl_lane_adjoint";
-    return field_config(c, sched, group, &field) ? "sodecl_field_adjoint" : "sodecl_group_adjoint";
-}
-
 }  // namespace
 
 extern "C" {
@@ -98,7 +91,7 @@ int sodecl_run_device_checkpointed(sodecl_ctx* c, double* t0, double* y0, const 
     std::shared_ptr<Program> prog;
     if (check_adjoint(c, sched, group, block)) prog = get_program(c, sched, group, block, kAdjointDefines);
     if (prog)
-        prog->get(adjoint_kernel(c, sched, group));
+        prog->get(prog->key.adjoint_kernel);
     else
         c->last_error = before;
     return 1;
@@ -126,18 +119,13 @@ int launch_adjoint(sodecl_ctx* c, const double* ckpt_t, const double* ckpt_y, co
                            "(sodecl_run_device_checkpointed) loads it");
         return 0;
     }
-    const char* kname = adjoint_kernel(c, sched, group);
-    hipFunction_t fn = prog->get(kname);
-    if (!fn) return fail(c, std::string("kernel ") + kname + " missing from the program");
+    hipFunction_t fn = prog->get(prog->key.adjoint_kernel);
+    if (!fn) return fail(c, std::string("kernel ") + prog->key.adjoint_kernel + " missing from the program");
     const long steps = total_steps(c);
     if (steps > 2147483647L) return fail(c, "too many steps");
     int orbits = c->orbits, nsteps = (int)steps, every = ckpt_every;
-    FieldConfig field;
-    if (field_config(c, sched, group, &field)) {
-        block = field.block;
-        group = field.lanes;
-    }
-    const int opb = implicit(c) ? block : block / group;
+    block = prog->key.threads;
+    const int opb = block / prog->key.orbit_lanes;
     const unsigned grid = (unsigned)((orbits + opb - 1) / opb);
     void* args[] = {(void*)&ckpt_t, (void*)&ckpt_y, (void*)&params, (void*)&cot, &grad_y0, &grad_params,
                     &work, &orbits, &nsteps, &every, &stored};

@@ -123,9 +123,12 @@ ProgramKey make_key(const sodecl_ctx* ctx, int schedule, int group, int block, c
     // sizes of 128 and 512 lanes).
     FieldConfig field;
     const bool in_field = field_config(ctx, schedule, group, &field);
-    k.noise_lanes = noise_lanes(ctx, schedule, block);
-    const int per_orbit = in_field ? field.lanes : schedule == 2 || schedule == 4 ? std::max(group, 1) : k.noise_lanes;
-    const long lanes = (long)ctx->orbits * per_orbit;
+    k.noise_lanes = in_field ? 1 : noise_lanes(ctx, schedule, block);
+    k.orbit_lanes = in_field ? field.lanes : schedule == 2 || schedule == 4 ? std::max(group, 1) : k.noise_lanes;
+    k.threads = in_field ? field.block : block;
+    k.kernel = in_field ? "sodecl_field" : schedule == 2 ? "sodecl_group" : schedule == 4 ? "sodecl_team" : "sodecl_lane";
+    k.adjoint_kernel = in_field ? "sodecl_field_adjoint" : schedule == 2 ? "sodecl_group_adjoint" : "sodecl_lane_adjoint";
+    const long lanes = (long)ctx->orbits * k.orbit_lanes;
     k.field_lanes = field.lanes;
     k.field_cpl = field.cpl;
     k.field_block = field.block;
@@ -138,13 +141,23 @@ ProgramKey make_key(const sodecl_ctx* ctx, int schedule, int group, int block, c
     return k;
 }
 
+// The name of a program among its context's: every field of its key that options
+// may change without dropping the programs (sodecl_set_options), so that two
+// texts never share one.
+std::string program_name(const ProgramKey& k)
+{
+    char name[128];
+    std::snprintf(name, sizeof name, "%d:%d:%d:%d:%d:%d:%d:%d:%d:", k.schedule, k.group, k.block, k.noise_lanes,
+                  k.field_lanes, k.field_cpl, k.field_block, k.use_pairs, k.one_wave_per_simd);
+    return name + k.extra_defines;
+}
+
 std::shared_ptr<Program> get_program(sodecl_ctx* ctx, int schedule, int group, int block, const std::string& extra)
 {
-    std::ostringstream name;
-    name << schedule << ":" << group << ":" << block << ":" << extra;
-    auto it = ctx->programs.find(name.str());
+    const ProgramKey key = make_key(ctx, schedule, group, block, extra);
+    const std::string name = program_name(key);
+    auto it = ctx->programs.find(name);
     if (it != ctx->programs.end()) return it->second;
-    ProgramKey key = make_key(ctx, schedule, group, block, extra);
     std::string text = assemble_program(ctx->system_source, key, ctx->features);
     ctx->last_program = text;
     auto prog = std::make_shared<Program>();
@@ -157,15 +170,15 @@ std::shared_ptr<Program> get_program(sodecl_ctx* ctx, int schedule, int group, i
     if (!hip_ok(ctx, hipSetDevice(ctx->device), "hipSetDevice")) return nullptr;
     if (!hip_ok(ctx, hipModuleLoadData(&prog->module, prog->code.data()), "hipModuleLoadData")) return nullptr;
     prog->device = ctx->device;
-    ctx->programs[name.str()] = prog;
+    prog->key = key;
+    prog->name = name;
+    ctx->programs[name] = prog;
     return prog;
 }
 
 std::shared_ptr<Program> find_program(sodecl_ctx* ctx, int schedule, int group, int block, const std::string& extra)
 {
-    std::ostringstream name;
-    name << schedule << ":" << group << ":" << block << ":" << extra;
-    auto it = ctx->programs.find(name.str());
+    auto it = ctx->programs.find(program_name(make_key(ctx, schedule, group, block, extra)));
     return it != ctx->programs.end() ? it->second : nullptr;
 }
 
@@ -460,26 +473,13 @@ int enqueue(sodecl_ctx* c, const LaunchCfg& cfg, double* t, double* y, const dou
 {
     auto prog = get_program(c, cfg.schedule, cfg.group, cfg.block);
     if (!prog) return 0;
-    FieldConfig field;
-    const bool in_field = field_config(c, cfg.schedule, cfg.group, &field);
-    const char* kname = in_field ? "sodecl_field"
-                                 : cfg.schedule == 2 ? "sodecl_group" : (cfg.schedule == 4 ? "sodecl_team" : "sodecl_lane");
-    hipFunction_t fn = prog->get(kname);
-    if (!fn) return fail(c, std::string("kernel ") + kname + " missing from the program");
+    hipFunction_t fn = prog->get(prog->key.kernel);
+    if (!fn) return fail(c, std::string("kernel ") + prog->key.kernel + " missing from the program");
     // the first norbits orbits only (the rest are the host share's)
     int orbits = norbits >= 0 ? norbits : c->orbits;
-    unsigned grid, block = (unsigned)cfg.block;
-    if (in_field) {
-        const int opb = field.block / field.lanes;
-        grid = (unsigned)((orbits + opb - 1) / opb);
-        block = (unsigned)field.block;
-    } else if (cfg.schedule == 2 || cfg.schedule == 4) {
-        const int opb = cfg.block / cfg.group;
-        grid = (unsigned)((orbits + opb - 1) / opb);
-    } else {
-        const int opb = cfg.block / noise_lanes(c, cfg.schedule, cfg.block);
-        grid = (unsigned)((orbits + opb - 1) / opb);
-    }
+    const unsigned block = (unsigned)prog->key.threads;
+    const int opb = prog->key.threads / prog->key.orbit_lanes;
+    const unsigned grid = (unsigned)((orbits + opb - 1) / opb);
     if (!ckpt_y || ckpt_every <= 0) {
         ckpt_y = nullptr;
         ckpt_t = nullptr;
@@ -1013,14 +1013,14 @@ int run_device_impl(sodecl_ctx* c, double* t0, double* y0, const double* params,
     // Several launches (segments_per_launch set): record the sequence once
     // as a hipGraph on the context's stream and replay it on the caller's
     // stream; the recording is reused while pointers and shape stay the same.
+    // compile before recording: no JIT inside a capture
+    const auto prog = get_program(c, cfg.schedule, cfg.group, cfg.block);
+    if (!prog) return 0;
     std::ostringstream key;
     key << (void*)t0 << (void*)y0 << (const void*)params << (void*)counters << (void*)traj << (void*)ckpt_t
-        << (void*)ckpt_y << (void*)stage_ws << ":" << ckpt_every << ":" << launches << ":" << per << ":" << cfg.schedule << ":"
-        << cfg.group << ":" << cfg.block;
+        << (void*)ckpt_y << (void*)stage_ws << ":" << ckpt_every << ":" << launches << ":" << per << ":" << prog->name;
     if (c->graph_key != key.str() || !c->graph_exec) {
         drop_graph(c);
-        // compile before recording: no JIT inside a capture
-        if (!get_program(c, cfg.schedule, cfg.group, cfg.block)) return 0;
         if (!hip_ok(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture"))
             return 0;
         int ok = enqueue_all(c->stream);

@@ -70,6 +70,11 @@ struct ProgramKey {
     int library_sin = 0;         // sin() in the system source: 0 sodecl_sin, 1 the device library's
     int library_exp = 0;         // exp() in the system source: 0 sodecl_exp, 1 the device library's
     std::string extra_defines;   // additional "#define" lines (adjoint, batch)
+    // How the program's kernels are launched: names, lanes per orbit, threads per block.
+    const char* kernel = "sodecl_lane";
+    const char* adjoint_kernel = "sodecl_group_adjoint";
+    int orbit_lanes = 1;
+    int threads = 128;
 };
 
 // printf("%g") of dt, as the reference's double2string (sodeclmgr.cpp:356-367).
@@ -86,8 +91,11 @@ std::string assemble_host_program(const std::string& system_source, const Progra
 std::string assemble_batch_program(const std::string& system_source, const ProgramKey& key, const PluginFeatures& f,
                                    const std::vector<BatchShape>& classes);
 
-// A compiled and loaded program.
+// A compiled and loaded program.  Launches take their geometry from its key,
+// never from options that may have changed since it was assembled.
 struct Program {
+    ProgramKey key;
+    std::string name;   // its key in the context's programs
     std::vector<char> code;
     hipModule_t module = nullptr;
     int device = -1;
@@ -150,7 +158,7 @@ struct sodecl_ctx {
     size_t stage_capacity = 0;
     hipEvent_t ev_start = nullptr, ev_stop = nullptr;
 
-    // programs: one per (schedule, group, block)
+    // programs, by everything that varies among a context's (program_name)
     std::map<std::string, std::shared_ptr<sodecl_amd::Program>> programs;
     int used_schedule = 0, used_group = 0, used_block = 0;
     bool tuning = false;            // the autotuner is timing its candidates
