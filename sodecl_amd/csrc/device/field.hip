@@ -123,11 +123,13 @@ SODECL_INLINE void sodecl_field_sums(int lane, const double (&phi)[SODECL_FC][SO
 }
 
 // Features, their sums, and the drift of this lane's components at x.
-// The features come from the copy of the plugin whose sincos() gives NaN
-// where the library's is needed (sodecl_sincos_marked): no branch or library
-// code per component, one test of the sums per drift.  Sums that are not
-// numbers send the orbit's features through the plugin as it stands, one
-// component at a time.
+// A source that defines SODE_FIELD_MARKED_SINCOS promises that a NaN sine from
+// any sincos() of its sode_field makes a sum NaN (no comparison, selection,
+// minimum or maximum takes it in between).  Its features come from a copy of
+// the source whose sincos() gives a NaN sine where the library's function is
+// needed (sodecl_sincos_marked): no branch or library code per component, one
+// test of the sums per drift.  Sums that are not numbers send the orbit's features
+// through the source as it stands, one component at a time.
 SODECL_INLINE void sodecl_field_eval(double t, const double (&x)[SODECL_FC], sodecl_field_params& pp, int lane,
                                      double (&phi)[SODECL_FC][SODE_FIELDS], double (&sum)[SODE_FIELDS],
                                      double (&f)[SODECL_FC])

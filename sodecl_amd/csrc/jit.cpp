@@ -228,12 +228,13 @@ std::string assemble_program(const std::string& system_source, const ProgramKey&
     o << system_source << "\n";
     o << system_end(k);
     if (k.field_lanes > 0 && !k.library_sin) {
-        // the same source once more, its sincos() marking what it does not
-        // cover instead of branching to the library (device/field.hip)
-        o << "#define SODECL_FIELD_MARKED 1\nnamespace sodecl_marked {\n";
+        // where the source allows it: the same source once more, its sincos()
+        // marking what it does not cover instead of branching to the library
+        // (device/field.hip)
+        o << "#ifdef SODE_FIELD_MARKED_SINCOS\n#define SODECL_FIELD_MARKED 1\nnamespace sodecl_marked {\n";
         o << "#define sin sodecl_sin\n#define sincos sodecl_sincos_marked\n"
           << (k.library_exp ? "" : "#define exp sodecl_exp\n") << "#pragma clang fp reciprocal(on)\n";
-        o << "#line 1 \"system.cl\"\n" << system_source << "\n" << system_end(k) << "}\n";
+        o << "#line 1 \"system.cl\"\n" << system_source << "\n" << system_end(k) << "}\n#endif\n";
     }
     o << "#pragma clang force_cuda_host_device end\n";
     o << "#line 1 \"integrators.hip\"\n";

@@ -166,6 +166,8 @@ void sode_system_vjp_group(double t, double x[_numeq_], double lam[_numeq_], dou
  * the same size as the rounding of w_i and below that of the states (which
  * grow with t), so trajectories keep the accuracy of the pairwise sums. */
 #define SODE_FIELDS 2
+/* The sine of the sincos() below is summed as it is: a NaN arrives in the sum. */
+#define SODE_FIELD_MARKED_SINCOS 1
 /* K is shared, w_i and (SDE form) the noise amplitude are component i's own. */
 #define SODE_FIELD_SHARED 1
 #define SODE_FIELD_OWN (_numnoi_ > 0 ? 2 : 1)
