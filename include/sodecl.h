@@ -59,7 +59,10 @@ enum sodecl_schedule {
                                   and the system is large enough, else team for Euler and RK4 with a
                                   plugin that has the entry point and few orbits, else lane; timed
                                   choice (team included) when autotune is on */
-    SODECL_SCHEDULE_LANE = 1,  /* one orbit per lane, state in registers */
+    SODECL_SCHEDULE_LANE = 1,  /* one orbit per lane, state in registers; Euler-Maruyama launches that
+                                  would leave SIMDs idle (1 to 16 noises) take up to 16 lanes per
+                                  orbit, each with the whole state: together they draw the noise, and
+                                  in pairs evaluate the plugin's sode_system_team, if it has one */
     SODECL_SCHEDULE_GROUP = 2, /* group_size lanes per orbit, stage vectors in LDS */
     SODECL_SCHEDULE_PLAIN = 3, /* the reference's launch design: one launch per ksteps
                                   segment with a blocking state read-back before each */

@@ -337,8 +337,8 @@ SODECL_INLINE int sodecl_lane_step(double t, double* y, double* yout, double* p)
 // together, and once every SODECL_NL steps lane j draws the noise of step j
 // ahead (Threefry counters as in sequence) into LDS, from where every lane
 // reads the current step's.  All of them carry the same state with the same
-// bits; lane 0 stores it.  Where the plugin has a team entry point they share
-// the drift's costly terms too (5000 oculomotor orbits x 1000 steps: 746 us on
+// bits; lane 0 stores it.  Where the plugin has a team entry point each pair of
+// them shares the drift's costly terms too (5000 oculomotor orbits x 1000 steps: 746 us on
 // one lane, 323 with the noise shared, 297 with four steps per block, 252 with
 // the drift shared).
 #ifndef SODECL_NL
@@ -355,7 +355,7 @@ SODECL_INLINE void sodecl_em_step(double& t, double* y, double* yn, double* p, d
 {
     double st[_numeq_];
 #ifdef SODECL_NOISE_TEAM
-    sode_system_team(t, y, yn, p);   // an orbit's lanes share the drift's costly terms as well
+    sode_system_team(t, y, yn, p);   // pairs of an orbit's lanes share the drift's costly terms as well
 #else
     sode_system(t, y, yn, p);
 #endif

@@ -119,11 +119,12 @@ __device__ inline double sodecl_group_sum(double v)
 //   sodecl_group_xor(v, m)  v of team lane sodecl_lane() ^ m (m < G)
 // These exist only in device code compiled for the team schedule, and for
 // Euler-Maruyama launches of the lane schedule whose orbits have several lanes
-// (SODECL_TEAM_API is defined there).
+// (SODECL_TEAM_API is defined there).  The lanes of such an orbit are teams of
+// two, as in an automatic team launch: a source may be written for pairs.
 #if SODECL_SCHEDULE == 4
 #define SODECL_TEAM_LANES SODECL_GROUP
 #elif SODECL_SCHEDULE == 1 && defined(SODECL_NOISE_TEAM)
-#define SODECL_TEAM_LANES SODECL_NL
+#define SODECL_TEAM_LANES 2
 #endif
 #ifdef SODECL_TEAM_LANES
 __device__ inline int sodecl_group_size() { return SODECL_TEAM_LANES; }
