@@ -264,11 +264,15 @@ sodecl_field(double* __restrict__ t_state, double* __restrict__ y_state, const d
     double cnt = active ? counters[orbit] : 0.0;
     const double dtsqrt = sqrt(_m_dt_);
     // Counters that stay whole numbers below 2^53 advance as 64-bit integers
-    // (the doubles' sums are exact there); any other counter goes through the
-    // double arithmetic of each call.
-    const double last = cnt + (double)nseg * (double)_numsteps_ * (double)SODECL_CALLS;
-    const bool whole = __all(cnt >= 0.0 && last < 0x1p53 && cnt == (double)(sodecl_u64)cnt);
-    sodecl_u64 word = whole ? (sodecl_u64)cnt : 0;
+    // (the doubles' sums are exact there); any other counter takes the
+    // reference's addition of each call.
+    const long long all_calls = (long long)nseg * _numsteps_ * SODECL_CALLS;
+    const bool whole = sodecl_counters_whole(cnt, (double)all_calls);
+    const double after = sodecl_counter_after(cnt, all_calls, whole);
+    // this lane's next call: its pair's, of the next step from odd lanes with
+    // one component per lane
+    cnt = sodecl_counter_after(cnt, SODECL_FC == 1 ? (lane >> 1) + ((lane & 1) ? SODECL_CALLS : 0) : lane * SODECL_FC / 2, whole);
+    sodecl_u64 word = sodecl_counter_word(cnt);
     (void)stage_ws;
     (void)ws_steps;
 #if SODECL_FC == 1
@@ -304,17 +308,21 @@ sodecl_field(double* __restrict__ t_state, double* __restrict__ y_state, const d
             }
             const int end = it + run;
 #if SODECL_IS_SDE
-            for (; it < end; ++it, ++g) {
+            // (two copies of the step: the branch in one cost 1.3%)
+            const auto step = [&](const bool ints) __attribute__((always_inline)) {
                 double z[SODECL_FC];
 #if SODECL_FC == 1
                 // Lane l draws call l / 2 of this step (l even) or of the next
                 // one (l odd): each lane of a call's pair keeps its half of the
                 // step it drew and swaps the other.
                 if (!drawn) {
-                    const int k = (lane >> 1) + ((lane & 1) ? SODECL_CALLS : 0);
                     double z0, z1;
-                    sodecl_noise_pair(orbit, whole ? word + (sodecl_u64)k : sodecl_counter_word(cnt + (double)k),
-                                      dtsqrt, &z0, &z1);
+                    sodecl_noise_pair(orbit, word, dtsqrt, &z0, &z1);
+                    word += 2 * SODECL_CALLS;
+                    if (!ints) {
+                        cnt = sodecl_counter_after(cnt, 2 * SODECL_CALLS, false);
+                        word = sodecl_counter_word(cnt);
+                    }
                     // (lanes l and l ^ 1 are neighbours in every mapping)
                     const double other = sodecl_dpp<SODECL_DPP_XOR1>((lane & 1) ? z0 : z1);
                     z[0] = (lane & 1) ? other : z0;
@@ -324,18 +332,28 @@ sodecl_field(double* __restrict__ t_state, double* __restrict__ y_state, const d
                 }
                 drawn = !drawn;
 #else
+                sodecl_u64 w[SODECL_FC / 2];
 #pragma unroll
-                for (int c = 0; c < SODECL_FC; c += 2) {
-                    const int k = (lane * SODECL_FC + c) / 2;
-                    sodecl_noise_pair(orbit, whole ? word + (sodecl_u64)k : sodecl_counter_word(cnt + (double)k),
-                                      dtsqrt, &z[c], &z[c + 1]);
+                for (int c = 0; c < SODECL_FC / 2; ++c) w[c] = word + (sodecl_u64)c;
+                word += SODECL_CALLS;
+                if (!ints) {
+#pragma unroll
+                    for (int c = 0; c < SODECL_FC / 2; ++c) {
+                        w[c] = sodecl_counter_word(cnt);
+                        cnt = cnt + 1;
+                    }
+                    cnt = sodecl_counter_after(cnt, SODECL_CALLS - SODECL_FC / 2, false);
                 }
+#pragma unroll
+                for (int c = 0; c < SODECL_FC; c += 2) sodecl_noise_pair(orbit, w[c / 2], dtsqrt, &z[c], &z[c + 1]);
 #endif
                 sodecl_field_step(t, y, pp, lane, z);
-                cnt = cnt + (double)SODECL_CALLS;
-                word += SODECL_CALLS;
                 t = t + _m_dt_;
-            }
+            };
+            if (whole)
+                for (; it < end; ++it, ++g) step(true);
+            else
+                for (; it < end; ++it, ++g) step(false);
 #else
             if (stage_ws) {
                 const size_t rows = (size_t)orbits * (size_t)ws_steps;
@@ -380,7 +398,7 @@ sodecl_field(double* __restrict__ t_state, double* __restrict__ y_state, const d
         if (lane == 0) {
             t_state[orbit] = t;
 #if SODECL_IS_SDE
-            counters[orbit] = cnt;
+            counters[orbit] = after;
 #endif
         }
     }

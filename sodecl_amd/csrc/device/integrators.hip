@@ -90,6 +90,23 @@ SODECL_INLINE sodecl_u64 sodecl_counter_word(double c)
 #define SODECL_RNG_KEY0 0ull
 #define SODECL_RNG_KEY1 0xf00dcafeull
 
+#if !defined(SODECL_HOST_BUILD)
+// The counter after k calls.  The reference adds 1 per call
+// (stochastic_solver_caller.cl:49-66), which rounds for fractions and stays
+// put from 2^53 on: one addition of k only where every counter of the wavefront
+// stays a whole number below 2^53 for all the launch's calls (whole).
+SODECL_INLINE double sodecl_counter_after(double c, long long k, bool whole)
+{
+    if (whole) return c + (double)k;
+    for (long long j = 0; j < k; ++j) c = c + 1;
+    return c;
+}
+SODECL_INLINE bool sodecl_counters_whole(double c, double calls)
+{
+    return __all(c >= 0.0 && c + calls < 0x1p53 && c == (double)(sodecl_u64)c);
+}
+#endif
+
 // One Box-Muller pair scaled by sqrt(dt) (stochastic_solver_caller.cl:54-65),
 // with the logarithm, sine and cosine specialised to the uniforms' ranges
 // (gauss.hip).
@@ -389,6 +406,9 @@ SODECL_INLINE void sodecl_lane_orbit(int i, int sub, double* buffer, double* __r
     const int calls = (int)ceilf((float)((float)(_numnoi_) * 0.5));
     double noise[SODECL_NNOI_ALLOC];
 #if SODECL_NL > 1
+    const long long all_calls = (long long)nseg * _numsteps_ * SODECL_CALLS;
+    const bool whole = sodecl_counters_whole(cnt, (double)all_calls);
+    double call = sodecl_counter_after(cnt, sub * SODECL_CALLS, whole);   // of this lane's next draw
     int drawn = SODECL_NL;   // step of the buffer that comes next: none left
 #endif
 #endif
@@ -428,13 +448,14 @@ SODECL_INLINE void sodecl_lane_orbit(int i, int sub, double* buffer, double* __r
                 // the noise of the next SODECL_NL steps
                 if (drawn == SODECL_NL) {
                     sodecl_wave_sync();   // the buffer's last step has been read
-                    const double first = cnt + (double)(sub * SODECL_CALLS);
                     for (int in = 0; in < SODECL_CALLS; ++in) {
                         double z0, z1;
-                        sodecl_noise_pair(i, sodecl_counter_word(first + (double)in), dtsqrt, &z0, &z1);
+                        sodecl_noise_pair(i, sodecl_counter_word(call), dtsqrt, &z0, &z1);
+                        call = call + 1;
                         buffer[sub * _numnoi_ + 2 * in] = z0;
                         if (2 * in + 1 < _numnoi_) buffer[sub * _numnoi_ + 2 * in + 1] = z1;
                     }
+                    call = sodecl_counter_after(call, (SODECL_NL - 1) * SODECL_CALLS, whole);
                     sodecl_wave_sync();
                     drawn = 0;
                 }
@@ -443,7 +464,6 @@ SODECL_INLINE void sodecl_lane_orbit(int i, int sub, double* buffer, double* __r
                 const auto step = [&]() {
                     for (int in = 0; in < _numnoi_; ++in) noise[in] = buffer[drawn * _numnoi_ + in];
                     ++drawn;
-                    cnt = cnt + (double)calls;
                     sodecl_em_step(t, y, yn, p, noise);
                 };
 #if SODECL_STEP_BLOCKS
@@ -481,6 +501,9 @@ SODECL_INLINE void sodecl_lane_orbit(int i, int sub, double* buffer, double* __r
         }
     }
     if (sub != 0) return;
+#if SODECL_NL > 1
+    cnt = sodecl_counter_after(cnt, all_calls, whole);
+#endif
     if (traj && final_snap) {
         double* o = traj + (size_t)(s0 + nseg) * slab + i;
         SODECL_UNROLL
