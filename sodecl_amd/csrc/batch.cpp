@@ -119,6 +119,13 @@ int lanes_for(int neq, int rows)
     return lanes;
 }
 
+// LDS bytes of a wavefront's parameters (device/batch_class.hip, SODECL_PLDS).
+size_t param_lds(const sodecl_batch* b, const BatchShape& s)
+{
+    const size_t row = b->npar <= 8 ? 0 : s.window ? b->npar | 1 : b->npar;
+    return row * s.slots() * sizeof(double);
+}
+
 // Lanes per orbit and form of every size class.
 //
 // Windowed form (up to 512 equations), by the wavefronts per SIMD of the whole
@@ -142,6 +149,9 @@ int lanes_for(int neq, int rows)
 //  * from four on, eight rows, where instructions count (32768 orbits of 32, 128 and
 //    512 equations: 7.6 ms, against 8.1 ms with four and 8.8 ms with two).
 // A power of two of rows keeps the parity of a row's index known to the compiler.
+// More than eight parameters are in LDS, a row per orbit: an orbit gets more
+// lanes than its rows need where a wavefront's orbits would take more than 16
+// KiB (which lets ten wavefronts onto a CU).
 //
 // Through LDS: 16 lanes up to 32 equations, 32 up to 128, else 64; the
 // 128-equation class ran 2.5-3% faster on 32 lanes (four rows per lane, four
@@ -166,6 +176,7 @@ std::vector<BatchShape> batch_shapes(const sodecl_batch* b)
             s.rows = rows;
             while (s.rows < reach || lanes_for(neq, s.rows) > 64) s.rows *= 2;
             s.lanes = lanes_for(neq, s.rows);
+            while (s.lanes < 64 && param_lds(b, s) > 16 * 1024) s.lanes *= 2;
             s.waves = 4;
         } else {
             s.lanes = neq <= 32 ? 16 : neq <= 128 ? 32 : 64;
@@ -325,6 +336,8 @@ int sodecl_batch_setup(sodecl_batch* b, int orbits, const int* orbit_class, cons
         return bhip(b, hipMalloc(dst, bytes), what) &&
                bhip(b, hipMemcpy(*dst, src, bytes, hipMemcpyHostToDevice), what);
     };
+    // (the device's limit for a block: 160 KiB)
+    const size_t max_lds = 160 * 1024;
     for (int ci = 0; ci < nclass; ++ci) {
         auto& c = b->classes[ci];
         const std::string name = "sodecl_batch_" + std::to_string(ci);
@@ -335,8 +348,10 @@ int sodecl_batch_setup(sodecl_batch* b, int orbits, const int* orbit_class, cons
         // orbits per wavefront (batch_class.hip)
         const long n = c.shape.neq;
         const long tlen = c.shape.rows >= 2 ? (n + 15) / 16 * 16 : n;
-        const long per_orbit = (c.shape.window ? 0 : 4 * tlen) + (b->npar <= 8 ? 0 : b->npar);
-        c.lds_bytes = (size_t)(per_orbit * c.shape.slots()) * sizeof(double);
+        c.lds_bytes = param_lds(b, c.shape) + (c.shape.window ? 0 : (size_t)(4 * tlen * c.shape.slots()) * sizeof(double));
+        if (c.nitems > 0 && c.lds_bytes > max_lds)
+            return bfail(b, "a size class needs " + std::to_string(c.lds_bytes) + " bytes of LDS per wavefront (" +
+                                std::to_string(b->npar) + " parameters), more than a block can have");
         if (c.nitems > 0 &&
             !up((void**)&c.d_items, c.items.data(), c.items.size() * sizeof(int), "work items"))
             return 0;

@@ -361,7 +361,8 @@ __device__ SODECL_BATCH_ITEM_ATTR void sodecl_batch_item(const int* __restrict__
 #pragma unroll
     for (int k = 0; k < _numpar_; ++k) sh_p[k] = has ? params_all[(size_t)o * _numpar_ + k] : 0.0;
 #else
-    double* const sh_p = lds + (size_t)part * _numpar_;
+    // (an odd row length: orbits of a wavefront read different banks)
+    double* const sh_p = lds + (size_t)part * (_numpar_ | 1);
     for (int k = lane; k < _numpar_; k += SODECL_LPO) sh_p[k] = has ? params_all[(size_t)o * _numpar_ + k] : 0.0;
     sodecl_wave_sync();
 #endif
