@@ -451,9 +451,16 @@ bool field_config(const sodecl_ctx* c, int schedule, int group, FieldConfig* f)
         for (int l = lanes / 2; l >= 1 && cpl(l) <= 5; l /= 2)
             if (cost(l) < cost(lanes)) lanes = l;
     }
-    if (cpl(lanes) > 16) return false;
     int block = 256;
     while (block > std::max(lanes, 64) && ((long)c->orbits * lanes + block - 1) / block < device_cus(c)) block /= 2;
+    // the adjoint gathers an orbit's parameter gradients in LDS: smaller blocks,
+    // then more lanes per orbit, until a block's fit 64 KiB
+    if (!sde && c->features.field_vjp) {
+        const auto fits = [&] { return (long)(block / lanes) * c->npar * 8 <= 64 * 1024; };
+        while (!fits() && block > std::max(lanes, 64)) block /= 2;
+        while (!fits() && lanes < 64 && c->opts.group_size <= 0 && !c->tuned_schedule && !c->tuning) lanes *= 2;
+    }
+    if (cpl(lanes) > 16) return false;
     f->lanes = lanes;
     f->cpl = cpl(lanes);
     f->block = block;
