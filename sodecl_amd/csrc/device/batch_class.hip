@@ -267,7 +267,10 @@ SODECL_INLINE void sodecl_pivots_scaled(double* pa, double* pb, double* q)
     *pb = na ? __builtin_nan("") : __builtin_amdgcn_ldexp(fb, -__builtin_amdgcn_frexp_exp(a));
     *pa = nb ? __builtin_nan("") : __builtin_amdgcn_ldexp(fa, -__builtin_amdgcn_frexp_exp(b));
 }
-// Solves such a system.  The reciprocals come in pairs, 1/a = b/(ab) and
+// Solves such a system: every row as if it were uncoupled, then the coupled ones
+// from their neighbours' (uncoupled) values.  Which rows are coupled only saves
+// work here: a zero that is not seen as a constant at one of the tests costs a
+// product with it.  The reciprocals come in pairs, 1/a = b/(ab) and
 // 1/b = a/(ab): ten issue slots in place of fourteen (a reciprocal's estimate
 // takes four).  An orbit whose residual norm is no number gets no numbers (the
 // reference's sweep carries it through every row).  Against the general solve:
@@ -296,19 +299,19 @@ SODECL_INLINE void sodecl_two_level_solve(Lo lo, double (&di)[SODECL_BR], Up up,
 #pragma unroll
     for (int k = 0; k < P; ++k) q[k] = sodecl_rcp(q[k]);
     const auto inv = [&](int j) { return R > 1 ? di[(j ^ 1) % R] * q[j / 2] : q[0]; };
-    const auto leaf = [&](int j) { return sodecl_zero(up(j)) && sodecl_zero(lo(j)); };
+    double u[R];
 #pragma unroll
-    for (int j = 0; j < R; ++j)
-        if (leaf(j)) x[j] = v[j] * inv(j);
+    for (int j = 0; j < R; ++j) u[j] = v[j] * inv(j);
     double before = 0.0, after = 0.0;   // the neighbouring partitions' last and first unknown
-    if (!sodecl_zero(up(0))) before = sodecl_pcr_neighbour(x[R - 1], lane, 1, true);
-    if (!sodecl_zero(lo(R - 1))) after = sodecl_pcr_neighbour(x[0], lane, 1, false);
+    if (!sodecl_zero(up(0))) before = sodecl_pcr_neighbour(u[R - 1], lane, 1, true);
+    if (!sodecl_zero(lo(R - 1))) after = sodecl_pcr_neighbour(u[0], lane, 1, false);
 #pragma unroll
     for (int j = 0; j < R; ++j) {
-        if (!leaf(j)) {
+        x[j] = u[j];
+        if (!(sodecl_zero(up(j)) && sodecl_zero(lo(j)))) {
             double s = v[j];
-            if (!sodecl_zero(up(j))) s = s - up(j) * (j > 0 ? x[j - 1 < 0 ? 0 : j - 1] : before);
-            if (!sodecl_zero(lo(j))) s = s - lo(j) * (j + 1 < R ? x[j + 1 < R ? j + 1 : 0] : after);
+            if (!sodecl_zero(up(j))) s = s - up(j) * (j > 0 ? u[j - 1 < 0 ? 0 : j - 1] : before);
+            if (!sodecl_zero(lo(j))) s = s - lo(j) * (j + 1 < R ? u[j + 1 < R ? j + 1 : 0] : after);
             x[j] = s * inv(j);
         }
     }
