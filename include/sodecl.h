@@ -57,7 +57,10 @@ enum sodecl_output { SODECL_OUTPUT_NONE = 0, SODECL_OUTPUT_ARRAY = 1, SODECL_OUT
 enum sodecl_schedule {
     SODECL_SCHEDULE_AUTO = 0,  /* group when the plugin has per-component entry points
                                   and the system is large enough, else team for Euler and RK4 with a
-                                  plugin that has the entry point and few orbits, else lane; timed
+                                  plugin that has the entry point and few orbits, else lane; with a
+                                  plugin in field form (see pairwise) its kernel takes the group
+                                  schedule's place, and the lane schedule's for two to seven
+                                  components where group_size and block_size are 0 too; timed
                                   choice (team included) when autotune is on */
     SODECL_SCHEDULE_LANE = 1,  /* one orbit per lane, state in registers; Euler-Maruyama launches that
                                   would leave SIMDs idle (1 to 16 noises) take up to 16 lanes per
@@ -322,8 +325,17 @@ double sodecl_last_host_ms(const sodecl_ctx* ctx, int* host_orbits);
  * nseg ksteps segments, snapshots into traj[s0 ..][neq][orbits]. */
 size_t sodecl_host_library(sodecl_ctx* ctx, char* path, size_t capacity);
 
-/* Schedule, group size and block size the last run (or sodecl_compile_only) used. */
+/* Schedule, group size and block size chosen for the last run (or
+ * sodecl_compile_only). */
 int sodecl_get_launch_config(const sodecl_ctx* ctx, int* schedule, int* group_size, int* block_size);
+
+/* What that run launched: its kernel (a static string; sodecl_field is the field
+ * form, which replaces the group schedule's kernel and, below eight components,
+ * the automatic lane schedule's), lanes per orbit and threads per block.  The
+ * field form, and small Euler-Maruyama launches of the lane schedule, choose
+ * these themselves. */
+int sodecl_get_launch_geometry(const sodecl_ctx* ctx, const char** kernel, int* lanes_per_orbit,
+                               int* threads_per_block);
 
 /* What the autotuner measured (candidate: time of one ksteps segment), or
  * "cached" when the choice came from its on-disk cache; empty without it. */

@@ -261,6 +261,13 @@ public:
         sodecl_get_launch_config(ctx_, &s, &g, &b);
         return py::make_tuple(s, g, b);
     }
+    py::tuple launch_geometry()
+    {
+        const char* kernel = "";
+        int lanes = 0, threads = 0;
+        sodecl_get_launch_geometry(ctx_, &kernel, &lanes, &threads);
+        return py::make_tuple(kernel, lanes, threads);
+    }
     double last_kernel_ms() const { return sodecl_last_kernel_ms(ctx_); }
     py::tuple host_stats() const
     {
@@ -428,6 +435,7 @@ PYBIND11_MODULE(sodecl_interface, m)
         .def("counters", &Session::get_counters)
         .def("newton_updates", &Session::newton_updates)
         .def("launch_config", &Session::launch_config)
+        .def("launch_geometry", &Session::launch_geometry)
         .def("last_kernel_ms", &Session::last_kernel_ms)
         .def("host_stats", &Session::host_stats)
         .def("last_runtime", &Session::last_runtime)

@@ -471,6 +471,17 @@ bool field_config(const sodecl_ctx* c, int schedule, int group, FieldConfig* f)
 
 namespace {
 
+// What sodecl_get_launch_config and sodecl_get_launch_geometry report.
+void note_launch(sodecl_ctx* c, const LaunchCfg& cfg, const ProgramKey& key)
+{
+    c->used_schedule = cfg.schedule;
+    c->used_group = cfg.group;
+    c->used_block = cfg.block;
+    c->used_kernel = key.kernel;
+    c->used_lanes = key.orbit_lanes;
+    c->used_threads = key.threads;
+}
+
 // Enqueues one launch of the chosen schedule: segments [s0, s0 + nseg) of the
 // trajectory buffer traj (snapshot rows), final snapshot when final_snap.
 int enqueue(sodecl_ctx* c, const LaunchCfg& cfg, double* t, double* y, const double* p, double* cnt, double* traj,
@@ -497,9 +508,7 @@ int enqueue(sodecl_ctx* c, const LaunchCfg& cfg, double* t, double* y, const dou
     if (!hip_ok(c, hipModuleLaunchKernel(fn, grid, 1, 1, block, 1, 1, 0, stream, args, nullptr),
                 "hipModuleLaunchKernel"))
         return 0;
-    c->used_schedule = cfg.schedule;
-    c->used_group = cfg.group;
-    c->used_block = cfg.block;
+    note_launch(c, cfg, prog->key);
     return 1;
 }
 
@@ -1347,6 +1356,15 @@ int sodecl_get_launch_config(const sodecl_ctx* c, int* schedule, int* group, int
     return 1;
 }
 
+int sodecl_get_launch_geometry(const sodecl_ctx* c, const char** kernel, int* lanes_per_orbit, int* threads_per_block)
+{
+    if (!c) return 0;
+    if (kernel) *kernel = c->used_kernel;
+    if (lanes_per_orbit) *lanes_per_orbit = c->used_lanes;
+    if (threads_per_block) *threads_per_block = c->used_threads;
+    return 1;
+}
+
 int sodecl_get_newton_updates(sodecl_ctx* c, long long* counts)
 {
     if (!c || !counts || !c->ready) return 0;
@@ -1360,10 +1378,8 @@ size_t sodecl_compile_only(sodecl_ctx* c, const char* arch)
 {
     if (!c) return 0;
     LaunchCfg cfg = choose_config(c);
-    c->used_schedule = cfg.schedule;   // reported by sodecl_get_launch_config
-    c->used_group = cfg.group;
-    c->used_block = cfg.block;
     ProgramKey key = sodecl_amd::make_key(c, cfg.schedule, cfg.group, cfg.block, std::string());
+    note_launch(c, cfg, key);
     size_t total = 0;
     std::vector<std::string> variants = {std::string()};
     // the adjoint program too, where this configuration supports one

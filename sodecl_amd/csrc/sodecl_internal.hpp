@@ -161,6 +161,8 @@ struct sodecl_ctx {
     // programs, by everything that varies among a context's (program_name)
     std::map<std::string, std::shared_ptr<sodecl_amd::Program>> programs;
     int used_schedule = 0, used_group = 0, used_block = 0;
+    const char* used_kernel = "";   // and what it launched
+    int used_lanes = 0, used_threads = 0;
     bool tuning = false;            // the autotuner is timing its candidates
     // autotuner result (schedule, group, block); tuned_schedule 0 = none
     int tuned_schedule = 0, tuned_group = 0, tuned_block = 0;
