@@ -210,7 +210,7 @@ sodecl_group_adjoint(const double* __restrict__ ckpt_t, const double* __restrict
 //   dL/dp += dt (df/dp)^T mu        at g (IE) or m (IM).
 // A^T mu = lam is solved by refinement with an approximate inverse,
 // mu += T^-1 (lam - A^T mu), until the residual's L1 norm is below 1e-15 of
-// lam's or after SODECL_NEWTON_MAXIT rounds.  Up to 12 equations T is A^T
+// lam's or after SODECL_NEWTON_MAXIT rounds.  Up to 10 equations T is A^T
 // itself, eliminated once per step (no pivoting: A is the identity and a
 // multiple of dt), whose rounds end after one or two; constant zeros of the
 // plugin's Jacobian drop out at compile time.  Beyond, T is the tridiagonal
@@ -239,8 +239,12 @@ sodecl_group_adjoint(const double* __restrict__ ckpt_t, const double* __restrict
 #endif
 #define SODECL_IMPLICIT_C (SODECL_SOLVER == 3 ? 1.0 : 0.50)
 
-// LU elimination of A^T in place of the tridiagonal band
-#define SODECL_ADJOINT_LU (_numeq_ <= 12)
+// LU elimination of A^T in place of the tridiagonal band.  A dense A^T, the
+// Jacobian and the factors leave the registers beyond ten equations: fit of
+// 8192 all-to-all coupled orbits, 40 midpoint steps, ms with the factors and
+// with the band: 9 equations 10.4 10.8, 10: 12.5 12.8, 11: 17.7 14.8, 12 (20000
+// orbits): 22.4 17.7.
+#define SODECL_ADJOINT_LU (_numeq_ <= 10)
 #if SODECL_ADJOINT_LU
 // lu = A^T = I - cdt J^T on entry; on return its factors (unit lower part
 // below the diagonal), the diagonal as reciprocals.
