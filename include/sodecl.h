@@ -247,8 +247,9 @@ int sodecl_adjoint_device_noalloc(sodecl_ctx* ctx, const double* ckpt_t, const d
  * every step's stage vectors to work (sodecl_stored_workspace_size doubles,
  * orbits x steps x (stages x neq + 1): 67 GB for 16384 orbits of a 64-equation
  * RK4 over 2000 steps); sodecl_adjoint_device_stored then sweeps backwards
- * from that workspace.  Gradients are bit-identical to the checkpointed
- * adjoint's. */
+ * from that workspace, with the arithmetic and row layout of the context's last
+ * stored run, also if options changed in between.  Gradients are bit-identical
+ * to the checkpointed adjoint's. */
 size_t sodecl_stored_workspace_size(const sodecl_ctx* ctx);
 int sodecl_run_device_stored(sodecl_ctx* ctx, double* t0, double* y0, const double* params, double* traj,
                              double* work, void* stream);

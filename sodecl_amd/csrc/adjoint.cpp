@@ -111,8 +111,9 @@ int launch_adjoint(sodecl_ctx* c, const double* ckpt_t, const double* ckpt_y, co
     if (!check_adjoint(c, sched, group, block)) return 0;
     if (stored && implicit(c)) return fail(c, "stored stage vectors are available for Euler and RK4 only");
     if (!hip_ok(c, hipSetDevice(c->device), "hipSetDevice")) return 0;
-    auto prog = loaded_only ? find_program(c, sched, group, block, kAdjointDefines)
-                            : get_program(c, sched, group, block, kAdjointDefines);
+    auto prog = loaded_only           ? find_program(c, sched, group, block, kAdjointDefines)
+                : stored && c->stored ? get_program(c, c->stored_key)
+                                      : get_program(c, sched, group, block, kAdjointDefines);
     if (!prog) {
         if (loaded_only)
             return fail(c, "the adjoint program is not loaded on this context: a checkpointed forward run "
@@ -195,7 +196,10 @@ int sodecl_run_device_stored(sodecl_ctx* c, double* t0, double* y0, const double
     int sched = 0, group = 0, block = 0;
     if (!check_adjoint(c, sched, group, block)) return 0;
     if (implicit(c)) return fail(c, "stored stage vectors are available for Euler and RK4 only");
-    return run_device_impl(c, t0, y0, params, nullptr, traj, nullptr, nullptr, 0, stream, work);
+    if (!run_device_impl(c, t0, y0, params, nullptr, traj, nullptr, nullptr, 0, stream, work)) return 0;
+    c->stored_key = make_key(c, sched, group, block, kAdjointDefines);
+    c->stored = true;
+    return 1;
 }
 
 int sodecl_adjoint_device_stored(sodecl_ctx* c, const double* params, const double* cot, double* grad_y0,

@@ -142,19 +142,24 @@ ProgramKey make_key(const sodecl_ctx* ctx, int schedule, int group, int block, c
 }
 
 // The name of a program among its context's: every field of its key that options
-// may change without dropping the programs (sodecl_set_options), so that two
-// texts never share one.
+// may change, so that two texts never share one (sodecl_set_options drops the
+// programs when the Newton options change).
 std::string program_name(const ProgramKey& k)
 {
-    char name[128];
-    std::snprintf(name, sizeof name, "%d:%d:%d:%d:%d:%d:%d:%d:%d:", k.schedule, k.group, k.block, k.noise_lanes,
-                  k.field_lanes, k.field_cpl, k.field_block, k.use_pairs, k.one_wave_per_simd);
+    char name[160];
+    std::snprintf(name, sizeof name, "%d:%d:%d:%d:%d:%d:%d:%d:%d:%d:%d:%d:", k.schedule, k.group, k.block, k.noise_lanes,
+                  k.field_lanes, k.field_cpl, k.field_block, k.use_pairs, k.one_wave_per_simd, k.fp_contract,
+                  k.library_sin, k.library_exp);
     return name + k.extra_defines;
 }
 
 std::shared_ptr<Program> get_program(sodecl_ctx* ctx, int schedule, int group, int block, const std::string& extra)
 {
-    const ProgramKey key = make_key(ctx, schedule, group, block, extra);
+    return get_program(ctx, make_key(ctx, schedule, group, block, extra));
+}
+
+std::shared_ptr<Program> get_program(sodecl_ctx* ctx, const ProgramKey& key)
+{
     const std::string name = program_name(key);
     auto it = ctx->programs.find(name);
     if (it != ctx->programs.end()) return it->second;

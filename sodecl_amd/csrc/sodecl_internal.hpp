@@ -163,6 +163,10 @@ struct sodecl_ctx {
     int used_schedule = 0, used_group = 0, used_block = 0;
     const char* used_kernel = "";   // and what it launched
     int used_lanes = 0, used_threads = 0;
+    // the adjoint program that reads the rows of the last sodecl_run_device_stored
+    // (their layout depends on the options of that run)
+    bool stored = false;
+    sodecl_amd::ProgramKey stored_key;
     bool tuning = false;            // the autotuner is timing its candidates
     // autotuner result (schedule, group, block); tuned_schedule 0 = none
     int tuned_schedule = 0, tuned_group = 0, tuned_block = 0;
@@ -210,6 +214,7 @@ int noise_lanes(const sodecl_ctx* c, int schedule, int block);
 // Program for the given schedule on the context's device (compiled on first use).
 std::shared_ptr<Program> get_program(sodecl_ctx* ctx, int schedule, int group, int block,
                                      const std::string& extra_defines = std::string());
+std::shared_ptr<Program> get_program(sodecl_ctx* ctx, const ProgramKey& key);
 // The program if it is already compiled and loaded on the context, else null
 // (no compilation, no module load).
 std::shared_ptr<Program> find_program(sodecl_ctx* ctx, int schedule, int group, int block,
