@@ -9,7 +9,7 @@
 // is integrated with O(N) work per drift instead of the O(N^2) of the
 // per-component and pairwise forms.  ps are the first SODE_FIELD_SHARED
 // parameters, po the SODE_FIELD_OWN parameters of component i,
-// po[k] = p[sode_field_own_param(i, k)].  Nothing passes through LDS:
+// po[k] = p[sode_field_own_param(i, k)].  The integration passes nothing through LDS:
 // SODECL_FL lanes share an orbit, lane l owns the SODECL_FC consecutive
 // components from l * SODECL_FC on, states and parameters in registers, sums
 // its features over them and then over the lanes by DPP moves, which leave
@@ -72,10 +72,9 @@ SODECL_INLINE void sodecl_field_load_params(const double* p, bool active, int la
 // ones (v_mfma_f64_4x4x4_4b_f64 holds four 4 x 4 matrices, matrix b on the
 // lanes with l / 4 mod 4 = b): the first adds the four lanes of a column, the
 // second the four columns, and lane moves join the orbit's two or four
-// matrices.  1500 orbits of 33 components on 32 lanes, 300 RK4 steps: 0.42 ->
-// 0.39 ms, 64 lanes 0.50 -> 0.44 ms; on 16 lanes the two products take as long
-// as the four levels of moves (0.79 ms for 16384 orbits of 64 components, 0.22
-// ms for the 1000 steps of 1024 orbits of 10) and lane moves stay.
+// matrices.  1500 orbits of 33 components on 32 lanes, 300 RK4 steps: 373 ->
+// 354 us; on 16 lanes the two products take as long as the four levels of moves
+// and lane moves stay.
 #define SODECL_FMATRIX (SODECL_FL >= 32)
 SODECL_INLINE int sodecl_field_lane(int tid)
 {

@@ -25,10 +25,15 @@
 
 // n / d correctly rounded for d in [1.7, 2.5] and |n| < 1/2, a multiple of
 // 2^-54; and the correctly rounded square root of a double in [2^-53, 128].
-// On the GPU they are the IEEE division's and square root's own refinement
-// steps, from the hardware's estimates on, without the scaling and the special
-// cases that these arguments do not need (the same bits, three and six
-// instructions fewer; tests compare both with the host's).
+// On the GPU they start from the hardware's estimates: the quotient by two
+// Newton-Raphson steps for the reciprocal and a correction by the quotient's exact
+// residual (P. Markstein, "Computation of elementary functions on the IBM RISC
+// System/6000 processor", IBM J. Res. Dev. 34, 1990), the root by a Goldschmidt
+// step for sqrt x and 1/(2 sqrt x) together and two corrections by the exact
+// residual x - g^2 (R. E. Goldschmidt, "Applications of division by convergence",
+// MIT, 1964; Markstein as above).  Neither needs scaling or special cases in these
+// ranges: three and six instructions fewer than the general operations, and the
+// same bits (tests compare both with the host's).
 SODECL_MATH_FN double sodecl_quotient_near(double n, double d)
 {
 #if defined(__HIP_DEVICE_COMPILE__)
