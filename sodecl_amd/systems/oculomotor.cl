@@ -117,9 +117,10 @@ void ocu_burst_pair(double x, double a, double b, double at, double bt, double e
      * multiply-add; a/b is written as the product with the reciprocal it
      * becomes where 1/b is at hand, which not every kernel's compiler sees.
      * The implicit solvers keep the form below, here and in ocu_rhs: the
-     * gradients of badly conditioned orbits amplify half an ulp of the drift
-     * a millionfold (8192 orbits fitted over 200 steps in 1.05 ms, against
-     * 1.03 with the rounded form, whose errors were up to 21 times larger) */
+     * gradients of badly conditioned orbits amplify the drift's rounding (8192
+     * orbits fitted over 200 midpoint steps: 1.05 ms; with the fused form 1.035
+     * ms, the largest gradient error against 64 bits 5.9e-13 instead of 2.6e-13
+     * on one set of inputs, 1.8e-13 instead of 2.9e-13 on another) */
     const int pos = x > 0;
     const double sat = fma(-at, es, at);
     const double ramp = (a * (1.0 / b)) * fabs(x) * er;
